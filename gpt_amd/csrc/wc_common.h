@@ -220,27 +220,34 @@ __device__ __forceinline__ C bload(wc_rsrc r, uint32_t voff, uint32_t soff) {
 
 typedef int wc_v4i __attribute__((ext_vector_type(4)));
 typedef int wc_v2i __attribute__((ext_vector_type(2)));
-template <typename C, int AUX = 0> struct bstore_t;
-template <int AUX> struct bstore_t<double2, AUX> {
-  static __device__ __forceinline__ void go(double2 v, wc_rsrc r, uint32_t voff, uint32_t soff) {
+
+// RB consecutive values (the right-hand sides r .. r + RB - 1 of one site and
+// component) as one memory access of 4, 8 or 16 bytes.  Raw buffer accesses
+// need dword alignment only, whatever their width, so r and N may be odd.
+template <typename S, int RB> struct rhs_pack {
+  S v[RB];
+};
+template <typename S, int RB, int AUX = 0>
+__device__ __forceinline__ rhs_pack<S, RB> bload_rhs(wc_rsrc r, uint32_t voff, uint32_t soff) {
+  using T = rhs_pack<S, RB>;
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8 || sizeof(T) == 16, "one access");
+  if constexpr (sizeof(T) == 16)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, AUX));
+  else if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, AUX));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, AUX));
+}
+template <typename S, int RB, int AUX = 0>
+__device__ __forceinline__ void bstore_rhs(rhs_pack<S, RB> v, wc_rsrc r, uint32_t voff, uint32_t soff) {
+  static_assert(sizeof(v) == 4 || sizeof(v) == 8 || sizeof(v) == 16, "one access");
+  if constexpr (sizeof(v) == 16)
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(wc_v4i, v), r, (int)voff, (int)soff, AUX);
-  }
-};
-template <int AUX> struct bstore_t<float2, AUX> {
-  static __device__ __forceinline__ void go(float2 v, wc_rsrc r, uint32_t voff, uint32_t soff) {
+  else if constexpr (sizeof(v) == 8)
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(wc_v2i, v), r, (int)voff, (int)soff, AUX);
-  }
-};
-template <int AUX> struct bstore_t<c2h, AUX> {
-  static __device__ __forceinline__ void go(c2h v, wc_rsrc r, uint32_t voff, uint32_t soff) {
+  else
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, (int)voff, (int)soff, AUX);
-  }
-};
-template <int AUX> struct bstore_t<c2b, AUX> {
-  static __device__ __forceinline__ void go(c2b v, wc_rsrc r, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, (int)voff, (int)soff, AUX);
-  }
-};
+}
 
 // compile-time tuning knobs of the hop kernel (defaults are the tuned values)
 #ifndef WC_LINK_AUX
@@ -248,12 +255,6 @@ template <int AUX> struct bstore_t<c2b, AUX> {
 #endif
 #ifndef WC_SPINOR_AUX
 #define WC_SPINOR_AUX 0  // cache policy of the neighbour-spinor gathers
-#endif
-#ifndef WC_NT_STORE
-#define WC_NT_STORE 1  // the hop output is not re-read by the hop: non-temporal stores
-#endif
-#ifndef WC_HOP_MINWAVES
-#define WC_HOP_MINWAVES 1  // occupancy hint (waves per SIMD) of the hop kernel
 #endif
 #ifndef WC_XCD_MAP
 #define WC_XCD_MAP 1  // XCD-contiguous block -> tile mapping

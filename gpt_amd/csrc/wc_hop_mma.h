@@ -315,7 +315,7 @@ __global__ __launch_bounds__(kMmaThreads, 4) void k_hop_mma(const HopLaunch a) {
           sum = fma((double)dv[k].y, (double)v[0][k].y, fma((double)dv[k].x, (double)v[0][k].x, sum));
         a.dots[h * N + rhs] = sum;
       }
-      store12_stream((SO *)a.out, g.Vh, h, rhs, N, v[0]);
+      store12_stream<SO, 1>((SO *)a.out, g.Vh, h, rhs, N, v);
     }
     __syncthreads();  // the next chunk overwrites lb
   }

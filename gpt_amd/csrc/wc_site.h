@@ -99,14 +99,29 @@ __device__ __forceinline__ void store12(S *f, long h, int r, int N, const C v[12
 #pragma unroll
   for (int k = 0; k < 12; ++k) p[(long)k * kBlk * N] = narrow<S>(v[k]);
 }
-// output of a hop: written once, not re-read by the kernel.  big: the field
-// exceeds one descriptor's 4 GB; the descriptor is then based at the 64-site
-// block of the wave's first active lane (every lane of a wave stores into
-// that block)
-template <typename S, typename C>
-__device__ __forceinline__ void store12_stream(S *f, long Vh, long h, int r, int N, const C v[12],
+// the right-hand sides r .. r + RB - 1 (all below N) of site h, one access
+// per component; f needs S's own alignment only
+template <typename S, int RB, typename C>
+__device__ __forceinline__ void load12_rhs(const S *f, long h, int r, int N, C v[RB][12]) {
+  const S *p = f + aidx_site(h, 12) * N + r;
+#pragma unroll
+  for (int k = 0; k < 12; ++k) {
+    rhs_pack<S, RB> q;
+    __builtin_memcpy(&q, p + (long)k * kBlk * N, sizeof q);
+#pragma unroll
+    for (int j = 0; j < RB; ++j) v[j][k] = widen(q.v[j]);
+  }
+}
+// output of a hop, right-hand sides r .. r + RB - 1 (all below N): written
+// once, not re-read by the kernel, one store per component.  Stored one by
+// one, the lanes of a wave would each fill part of a 64-byte segment per
+// store, and the non-temporal stores would write every segment RB times.
+// big: the field exceeds one descriptor's 4 GB; the descriptor is then based
+// at the 64-site block of the wave's first active lane (every lane of a wave
+// stores into that block)
+template <typename S, int RB, typename C>
+__device__ __forceinline__ void store12_stream(S *f, long Vh, long h, int r, int N, const C v[RB][12],
                                                bool big = false) {
-#if WC_NT_STORE
   wc_rsrc rs;
   uint32_t vo;
   if (big) {
@@ -119,11 +134,12 @@ __device__ __forceinline__ void store12_stream(S *f, long Vh, long h, int r, int
     vo = (uint32_t)(aidx_site(h, 12) * N + r) * (uint32_t)sizeof(S);
   }
 #pragma unroll
-  for (int k = 0; k < 12; ++k)
-    bstore_t<S, 2>::go(narrow<S>(v[k]), rs, vo, (uint32_t)(k * kBlk * N * sizeof(S)));
-#else
-  store12(f, h, r, N, v);
-#endif
+  for (int k = 0; k < 12; ++k) {
+    rhs_pack<S, RB> q;
+#pragma unroll
+    for (int j = 0; j < RB; ++j) q.v[j] = narrow<S>(v[j][k]);
+    bstore_rhs<S, RB, 2>(q, rs, vo, (uint32_t)(k * kBlk * N * sizeof(S)));
+  }
 }
 
 }  // namespace wck

@@ -62,6 +62,13 @@ __device__ __forceinline__ void accum_lower(C &a2, C &a3, const C c0, const C c1
   }
 }
 
+// third row = conj(row0 x row1) for SU(3)
+template <typename C> __device__ __forceinline__ void link_third_row(C u[9]) {
+  u[6] = cconj(csub(cmul(u[1], u[5]), cmul(u[2], u[4])));
+  u[7] = cconj(csub(cmul(u[2], u[3]), cmul(u[0], u[5])));
+  u[8] = cconj(csub(cmul(u[0], u[4]), cmul(u[1], u[3])));
+}
+
 // the link of direction (mu, fb) as the hop applies it: the third row
 // rebuilt for 12-real storage, the hop coefficient (and the boundary phase on
 // links that wrap around) folded in
@@ -71,12 +78,7 @@ __device__ __forceinline__ void prepare_link(const HopLaunch &a, int mu, int fb,
   using C = typename c2<R>::t;
   const Geom &g = a.g;
   const bool bnd = (fb == 0) ? (c[mu] == g.L[mu] - 1) : (c[mu] == 0);
-  if (NL == 6) {
-    // third row = conj(row0 x row1) for SU(3)
-    u[6] = cconj(csub(cmul(u[1], u[5]), cmul(u[2], u[4])));
-    u[7] = cconj(csub(cmul(u[2], u[3]), cmul(u[0], u[5])));
-    u[8] = cconj(csub(cmul(u[0], u[4]), cmul(u[1], u[3])));
-  }
+  if (NL == 6) link_third_row(u);
   const R coef = (R)(mu == 3 ? a.ct : a.cs);
   if (bnd) {
     C f = cmk<C>((R)(a.ph[mu][0]), (R)(fb == 0 ? a.ph[mu][1] : -a.ph[mu][1]));
@@ -277,6 +279,85 @@ __host__ __device__ inline bool xs_on(const HopLaunch &a) {
   return a.shape.ls == 2 && a.nrhs == 1 && a.shape.seg <= 1;
 }
 
+// What a hop does with the sums acc of site h, right-hand sides rb ..
+// rb + RB - 1: the epilogue's clover, axpy or diagonal term and inner product,
+// then the store.  get_y, get_dv: the operands a.y and a.dotv of the item,
+// fetched where they are used.  zb: the site lies on an open boundary.  cst (or null): the site's clover blocks in LDS, slot k
+// at cst[k * cstride] -- those of EPI_CLOV, or of EPI_DIAG without it.
+template <typename R, int EPI, int RB, typename SO, typename FY, typename FD>
+__device__ __forceinline__ void hop_epilogue(const HopLaunch &a, long h, int rb, bool zb,
+                                             const typename c2<R>::t *cst, long cstride,
+                                             typename c2<R>::t acc[RB][12], FY &&get_y, FD &&get_dv) {
+  using C = typename c2<R>::t;
+  const int N = a.nrhs;
+  if (zb) {
+#pragma unroll
+    for (int j = 0; j < RB; ++j)
+#pragma unroll
+      for (int k = 0; k < 12; ++k) acc[j][k] = cmk<C>(0, 0);
+  } else if (EPI & EPI_CLOV) {
+    if (cst) {
+      clov_apply_inplace_at<R, RB>(cst, cstride, acc);
+    } else if (a.clov && a.clov_roff) {
+      // one set of blocks per right-hand side (a batch of several masses)
+#pragma unroll
+      for (int j = 0; j < RB; ++j) {
+        C o[12];
+        clov_apply<R>((const C *)a.clov + a.clov_roff[rb + j], h, acc[j], o);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) acc[j][k] = o[k];
+      }
+    } else if (a.clov) {
+      clov_apply_inplace<R, RB>((const C *)a.clov, h, acc);
+    } else {
+#pragma unroll
+      for (int j = 0; j < RB; ++j)
+#pragma unroll
+        for (int k = 0; k < 12; ++k) acc[j][k] = cscale(acc[j][k], (R)a.clov_scalar);
+    }
+  }
+  if (EPI & EPI_DIAG) {
+    C y[RB][12];
+    get_y(y);
+    if (!zb) {
+      if ((EPI & EPI_CLOV) == 0 && cst) {
+        clov_apply_inplace_at<R, RB>(cst, cstride, y);
+      } else if (a.diag_clov) {
+        clov_apply_inplace<R, RB>((const C *)a.diag_clov, h, y);
+      } else {
+#pragma unroll
+        for (int j = 0; j < RB; ++j)
+#pragma unroll
+          for (int k = 0; k < 12; ++k) y[j][k] = cscale(y[j][k], (R)a.diag);
+      }
+#pragma unroll
+      for (int j = 0; j < RB; ++j)
+#pragma unroll
+        for (int k = 0; k < 12; ++k) acc[j][k] = cadd(acc[j][k], y[j][k]);
+    }
+  } else if (EPI & EPI_AXPY) {
+    C y[RB][12];
+    get_y(y);
+#pragma unroll
+    for (int j = 0; j < RB; ++j)
+#pragma unroll
+      for (int k = 0; k < 12; ++k) acc[j][k] = csub(y[j][k], acc[j][k]);
+  }
+  if (EPI & EPI_DOT) {
+    C dv[RB][12];
+    get_dv(dv);
+#pragma unroll
+    for (int j = 0; j < RB; ++j) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < 12; ++k)
+        s = fma((double)dv[j][k].y, (double)acc[j][k].y, fma((double)dv[j][k].x, (double)acc[j][k].x, s));
+      a.dots[h * N + rb + j] = s;
+    }
+  }
+  store12_stream<SO, RB>((SO *)a.out, a.g.Vh, h, rb, N, acc, a.big != 0);
+}
+
 // waves per SIMD the register allocation must allow: 4 for the FP32 hop
 // with one right-hand side per thread (<= 128 VGPRs), else 2 (<= 256; keeps
 // the compiler from parking accumulators in AGPRs at 1 wave)
@@ -380,70 +461,10 @@ __global__ __launch_bounds__(512, (hop_min_waves<R, RB>())) void k_hop(const Hop
                                                                    stage + sv, ns, xst, q0, xsn, (int)blockDim.x);
   // epilogue
   const bool zb = a.open_bc && (c[3] == 0 || c[3] == g.L[3] - 1);
-  if (zb) {
-#pragma unroll
-    for (int j = 0; j < RB; ++j)
-#pragma unroll
-      for (int k = 0; k < 12; ++k) acc[j][k] = cmk<C>(0, 0);
-  } else if (EPI & EPI_CLOV) {
-    if (LS && clov_staged) {
-      clov_apply_inplace_at<R, RB>(stage + 72 * ns + sv, (long)ns, acc);
-    } else if (a.clov && a.clov_roff) {
-      // one set of blocks per right-hand side (a batch of several masses)
-#pragma unroll
-      for (int j = 0; j < RB; ++j) {
-        C o[12];
-        clov_apply<R>((const C *)a.clov + a.clov_roff[rb + j], h, acc[j], o);
-#pragma unroll
-        for (int k = 0; k < 12; ++k) acc[j][k] = o[k];
-      }
-    } else if (a.clov) {
-      clov_apply_inplace<R, RB>((const C *)a.clov, h, acc);
-    } else {
-#pragma unroll
-      for (int j = 0; j < RB; ++j)
-#pragma unroll
-        for (int k = 0; k < 12; ++k) acc[j][k] = cscale(acc[j][k], (R)a.clov_scalar);
-    }
-  }
-  if (EPI & (EPI_DIAG | EPI_AXPY)) {
-    C y[RB][12];
-    load12_rhs<SI, RB>((const SI *)a.y, h, rb, N, y);
-    if (EPI & EPI_DIAG) {
-      if (!zb) {
-        if (a.diag_clov) {
-          clov_apply_inplace<R, RB>((const C *)a.diag_clov, h, y);
-        } else {
-#pragma unroll
-          for (int j = 0; j < RB; ++j)
-#pragma unroll
-            for (int k = 0; k < 12; ++k) y[j][k] = cscale(y[j][k], (R)a.diag);
-        }
-#pragma unroll
-        for (int j = 0; j < RB; ++j)
-#pragma unroll
-          for (int k = 0; k < 12; ++k) acc[j][k] = cadd(acc[j][k], y[j][k]);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < RB; ++j)
-#pragma unroll
-        for (int k = 0; k < 12; ++k) acc[j][k] = csub(y[j][k], acc[j][k]);
-    }
-  }
-  if (EPI & EPI_DOT) {
-    C v[RB][12];
-    load12_rhs<SI, RB>((const SI *)a.dotv, h, rb, N, v);
-#pragma unroll
-    for (int j = 0; j < RB; ++j) {
-      double s = 0.0;
-#pragma unroll
-      for (int k = 0; k < 12; ++k)
-        s = fma((double)v[j][k].y, (double)acc[j][k].y, fma((double)v[j][k].x, (double)acc[j][k].x, s));
-      a.dots[h * N + rb + j] = s;
-    }
-  }
-  store12_stream<SO, RB>((SO *)a.out, g.Vh, h, rb, N, acc, a.big != 0);
+  hop_epilogue<R, EPI, RB, SO>(
+      a, h, rb, zb, clov_staged ? stage + 72 * ns + sv : nullptr, (long)ns, acc,
+      [&](C y[RB][12]) { load12_rhs<SI, RB>((const SI *)a.y, h, rb, N, y); },
+      [&](C dv[RB][12]) { load12_rhs<SI, RB>((const SI *)a.dotv, h, rb, N, dv); });
 }
 
 // epilogues instantiated per storage: all of them in the working precision;

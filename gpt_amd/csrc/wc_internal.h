@@ -408,6 +408,9 @@ inline HopLaunch hop_args(const wc_operator *op, int nrhs, int pout, int dag, in
   a.halt = op->halt_cur;
   a.mma = mma_for(op, nrhs);
   a.clov_roff = clov_roff(op);
+  // a caller's shape is for the gathering kernel
+  const bool user = nrhs >= 1 && nrhs <= 64 && op->shape_user[nrhs];
+  a.march = user || a.shape.form == 2 ? 0 : a.shape.form == 1 ? 1 : 2;
   return a;
 }
 
@@ -551,7 +554,7 @@ inline void op_key(const wc_operator *op, int nrhs, std::vector<uintptr_t> &key)
                       (uintptr_t)clov_inv(op, 1), (uintptr_t)clov_roff(op), tmp(0), tmp(1), tmp(2), (uintptr_t)op->dots, (uintptr_t)op->partials, bits(op->diag), bits(op->cs), bits(op->ct), (uintptr_t)op->open_bc,
                       (uintptr_t)op->has_clover, (uintptr_t)sh.rb, (uintptr_t)sh.tpb, (uintptr_t)sh.occ,
                       (uintptr_t)sh.seg, (uintptr_t)sh.ls, (uintptr_t)op->bps, (uintptr_t)s16.rb, (uintptr_t)s16.tpb,
-                      (uintptr_t)s16.occ, (uintptr_t)s16.seg, (uintptr_t)s16.ls, (uintptr_t)mma_for(op, nrhs)})
+                      (uintptr_t)s16.occ, (uintptr_t)s16.seg, (uintptr_t)s16.ls, (uintptr_t)mma_for(op, nrhs), (uintptr_t)op->shape_user[nrhs], (uintptr_t)sh.form})
     key.push_back(v);
   for (int mu = 0; mu < 4; ++mu) {
     key.push_back(bits(op->p.boundary_phases[mu][0]));

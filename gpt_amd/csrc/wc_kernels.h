@@ -29,6 +29,7 @@ struct HopShape {
   int ls = 0;   // 1: a workgroup stages its sites' links (and EPI_CLOV blocks) in LDS once;
                 // 2 (one right-hand side): it stages the input spinors of its own half-site
                 // range, where the +-x and most +-y neighbours are
+  int form = 0; // hops that have a t-marching form: 0 by its rule, 1 the tuner found it faster, 2 slower
 };
 constexpr int kLdsPerCU = 160 * 1024;
 constexpr int kMaxStageBytes = 80 * 1024;  // largest LDS staging area of one workgroup
@@ -71,6 +72,9 @@ struct HopLaunch {
   int mma;           // 1: FP16-storage hops of 4k right-hand sides run on the matrix cores (k_hop_mma)
   const long *clov_roff; // non-null: right-hand side r uses the EPI_CLOV blocks at clov + clov_roff[r]
                          // (device array, complex elements; a batch of several masses), null: one set
+  int march;         // hops of many right-hand sides on the t-marching kernel (k_hop_march) where it
+                     // applies: 0 no, 1 yes, 2 by its rule of sizes
+  int march_segs;    // set by its launch: t-segments of the lattice
   int big;           // set by the launch: in or out exceeds one buffer descriptor's 4 GB, so
                      // gathers go through a descriptor based at the neighbours' t-slice and
                      // stores through one based at the wave's 64-site block
@@ -92,6 +96,9 @@ constexpr int kRedBlocks = 1024;  // fixed grid of the reduction kernels
 
 // returns false (nothing launched) for a shape outside the limits above
 template <typename R> bool hop(const HopLaunch &a, hipStream_t s);
+// the t-marching form (wc_hop_march.h): whether a launch has it (a.march set,
+// working precision, enough right-hand sides, ...); the shape is not used
+template <typename R> bool hop_march_applies(const HopLaunch &a);
 // the matrix-core form of the FP16-storage hop: hop_mma_applies says whether
 // the launch has that form (a.mma set, c2h input, N a multiple of 4, ...);
 // hop_mma launches it (false: not applicable or epilogue not instantiated)

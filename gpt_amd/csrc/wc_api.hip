@@ -698,6 +698,7 @@ static int tune_impl(wc_operator *op, int N, int reps, hipStream_t s, wck::HopSh
     HopLaunch a = hop_args<R>(op, N, 0, 0, op->has_clover ? wck::EPI_CLOV : 0, op->tmp[1], op->tmp[0]);
     a.clov = op->has_clover ? op->Ai[0] : nullptr;
     a.shape = sh;
+    a.split = 0;
     a.march = march;
     // shapes this device cannot launch, or whose staging area is too large
     if (!wck::hop<R>(a, s) || hipGetLastError() != hipSuccess) return WC_OK;

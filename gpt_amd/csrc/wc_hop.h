@@ -62,6 +62,24 @@ __device__ __forceinline__ void accum_lower(C &a2, C &a3, const C c0, const C c1
   }
 }
 
+// neighbour half-site of output half-site hh (coordinates c0..c3) in
+// direction dir = 2 mu + fb (fb 0: +mu, 1: -mu), periodic
+__device__ __forceinline__ uint32_t hop_neighbour(const Geom &g, uint32_t hh, int c0, int c1, int c2, int c3,
+                                                  int dir) {
+  const int mu = dir >> 1, fb = dir & 1;
+  if (mu == 0) {
+    const int xn = fb == 0 ? (c0 == g.L[0] - 1 ? 0 : c0 + 1) : (c0 == 0 ? g.L[0] - 1 : c0 - 1);
+    return hh - ((uint32_t)c0 >> 1) + ((uint32_t)xn >> 1);
+  }
+  const uint32_t st1 = (uint32_t)g.Lxh, st2 = st1 * (uint32_t)g.L[1], st3 = st2 * (uint32_t)g.L[2];
+  const uint32_t stride = mu == 1 ? st1 : (mu == 2 ? st2 : st3);
+  const int cm = mu == 1 ? c1 : (mu == 2 ? c2 : c3);
+  const int Lm = mu == 1 ? g.L[1] : (mu == 2 ? g.L[2] : g.L[3]);
+  const uint32_t wrap = (uint32_t)(Lm - 1) * stride;
+  if (fb == 0) return (cm == Lm - 1) ? hh - wrap : hh + stride;
+  return (cm == 0) ? hh + wrap : hh - stride;
+}
+
 // third row = conj(row0 x row1) for SU(3)
 template <typename C> __device__ __forceinline__ void link_third_row(C u[9]) {
   u[6] = cconj(csub(cmul(u[1], u[5]), cmul(u[2], u[4])));

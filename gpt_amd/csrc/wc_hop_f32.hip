@@ -7,12 +7,15 @@
 // iteration run, so no kernel of a captured run triggers a module load.
 #include "wc_hop.h"
 #include "wc_hop_march.h"
+#include "wc_hop_split.h"
 #include "wc_hop_mma.h"
 
 namespace wck {
 template <> bool hop_march_applies<float>(const HopLaunch &a) { return march_applies<float>(a); }
+template <> bool hop_split_applies<float>(const HopLaunch &a) { return split_applies<float>(a); }
 template <> bool hop<float>(const HopLaunch &a, hipStream_t s) {
   if (hop_mma_applies(a) && hop_mma(a, s)) return true;
+  if (split_applies<float>(a)) return hop_split<float>(a, s);
   if (march_applies<float>(a)) return hop_march<float>(a, s);
   return hop_launch<float>(a, s);
 }

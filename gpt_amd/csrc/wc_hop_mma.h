@@ -60,24 +60,6 @@ constexpr int kMmaChunk = 16;    // right-hand sides per pass: 4 column tiles of
 constexpr float kMmaHiScale = 256.0f;
 constexpr float kMmaLoScale = 2048.0f;
 
-// neighbour half-site of output half-site hh (coordinates c0..c3) in
-// direction dir = 2 mu + fb (fb 0: +mu, 1: -mu), periodic
-__device__ __forceinline__ uint32_t mma_neighbour(const Geom &g, uint32_t hh, int c0, int c1, int c2, int c3,
-                                                  int dir) {
-  const int mu = dir >> 1, fb = dir & 1;
-  if (mu == 0) {
-    const int xn = fb == 0 ? (c0 == g.L[0] - 1 ? 0 : c0 + 1) : (c0 == 0 ? g.L[0] - 1 : c0 - 1);
-    return hh - ((uint32_t)c0 >> 1) + ((uint32_t)xn >> 1);
-  }
-  const uint32_t st1 = (uint32_t)g.Lxh, st2 = st1 * (uint32_t)g.L[1], st3 = st2 * (uint32_t)g.L[2];
-  const uint32_t stride = mu == 1 ? st1 : (mu == 2 ? st2 : st3);
-  const int cm = mu == 1 ? c1 : (mu == 2 ? c2 : c3);
-  const int Lm = mu == 1 ? g.L[1] : (mu == 2 ? g.L[2] : g.L[3]);
-  const uint32_t wrap = (uint32_t)(Lm - 1) * stride;
-  if (fb == 0) return (cm == Lm - 1) ? hh - wrap : hh + stride;
-  return (cm == 0) ? hh + wrap : hh - stride;
-}
-
 // f * v for f in {1, -1, i, -i} on a complex FP16 pair held as one dword:
 // swap (f = +-i) takes (re, im) to (-im, re), neg negates both halves
 __device__ __forceinline__ uint32_t mma_times(uint32_t v, bool swap, bool neg) {
@@ -140,7 +122,7 @@ __global__ __launch_bounds__(kMmaThreads, 4) void k_hop_mma(const HopLaunch a) {
         const long h = site0 + s;
         int c[4];
         half_coords(g, h, a.pout, c);
-        const uint32_t nb = mma_neighbour(g, (uint32_t)h, c[0], c[1], c[2], c[3], dir);
+        const uint32_t nb = hop_neighbour(g, (uint32_t)h, c[0], c[1], c[2], c[3], dir);
         // h_su = p_su + f p_pt, the upper spin of (1 - S gamma_mu) psi
         const int S = ((fb == 0) != (DAG != 0)) ? 1 : -1;
         const int pt = mu < 2 ? 3 - su : 2 + su;

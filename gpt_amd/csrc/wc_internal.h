@@ -410,6 +410,7 @@ inline HopLaunch hop_args(const wc_operator *op, int nrhs, int pout, int dag, in
   a.clov_roff = clov_roff(op);
   // a caller's shape is for the gathering kernel
   const bool user = nrhs >= 1 && nrhs <= 64 && op->shape_user[nrhs];
+  a.split = user ? 0 : 1;
   a.march = user || a.shape.form == 2 ? 0 : a.shape.form == 1 ? 1 : 2;
   return a;
 }
@@ -431,6 +432,11 @@ inline void site_op(const wc_operator *op, int nrhs, int p, int inv, const void 
   double sc = inv ? 1.0 / op->diag : op->diag;
   wck::site_clover<R>(op->g, nrhs, p, B, sc, in, out, y, op->open_bc ? 1 : 0, s, half,
                       inv ? clov_roff(op) : nullptr);
+}
+
+// whether the launch itself writes dot_blocks' sums
+template <typename R> inline bool dots_summed(const HopLaunch &a) {
+  return a.nrhs == 1 && a.dot_partials && wck::hop_split_applies<R>(a);
 }
 
 // Mpc (which 0), Mpc^dag (1) or Mpc^dag Mpc (2) with D = pd on nrhs
@@ -468,10 +474,11 @@ inline int mpc_run(wc_operator *op, int nrhs, int pd, int which, void *out, cons
     b.y = src;
     b.dotv = dotv;
     b.dots = dots;
+    b.dot_partials = partials;
     b.half_in = b.half_out = half;
     if (half) b.shape = a.shape;
     WC_HOP(R, b, s);
-    if (which == 0 && dotv) wck::dot_blocks(op->g, nrhs, dots, partials, s, op->halt_cur);
+    if (which == 0 && dotv && !dots_summed<R>(b)) wck::dot_blocks(op->g, nrhs, dots, partials, s, op->halt_cur);
     src = dst_mpc;
   }
   if (which == 1 || which == 2) {
@@ -486,10 +493,11 @@ inline int mpc_run(wc_operator *op, int nrhs, int pd, int which, void *out, cons
     b.y = src;
     b.dotv = dotv;
     b.dots = dots;
+    b.dot_partials = partials;
     b.half_in = half;  // the product itself stays in the working precision
     if (half) b.shape = a.shape;
     WC_HOP(R, b, s);
-    if (dotv) wck::dot_blocks(op->g, nrhs, dots, partials, s, op->halt_cur);
+    if (dotv && !dots_summed<R>(b)) wck::dot_blocks(op->g, nrhs, dots, partials, s, op->halt_cur);
   }
   WC_LAUNCHED();
   return WC_OK;

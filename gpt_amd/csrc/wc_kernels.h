@@ -75,6 +75,9 @@ struct HopLaunch {
   int march;         // hops of many right-hand sides on the t-marching kernel (k_hop_march) where it
                      // applies: 0 no, 1 yes, 2 by its rule of sizes
   int march_segs;    // set by its launch: t-segments of the lattice
+  int split;         // 1: hops of few sites go to the kernel with one wave per direction (k_hop_split)
+  double *dot_partials;  // k_hop_split's EPI_DOT with one right-hand side: also the sums of dot_blocks
+                         // (or null)
   int big;           // set by the launch: in or out exceeds one buffer descriptor's 4 GB, so
                      // gathers go through a descriptor based at the neighbours' t-slice and
                      // stores through one based at the wave's 64-site block
@@ -99,6 +102,8 @@ template <typename R> bool hop(const HopLaunch &a, hipStream_t s);
 // the t-marching form (wc_hop_march.h): whether a launch has it (a.march set,
 // working precision, enough right-hand sides, ...); the shape is not used
 template <typename R> bool hop_march_applies(const HopLaunch &a);
+// whether the launch goes to k_hop_split (wc_hop_split.h), which writes dot_partials itself
+template <typename R> bool hop_split_applies(const HopLaunch &a);
 // the matrix-core form of the FP16-storage hop: hop_mma_applies says whether
 // the launch has that form (a.mma set, c2h input, N a multiple of 4, ...);
 // hop_mma launches it (false: not applicable or epilogue not instantiated)

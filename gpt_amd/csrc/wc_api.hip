@@ -345,12 +345,9 @@ static int cg_impl(wc_operator *op, int nrhs, int pd, void *x, const void *b, do
   op_key(op, N, key);
   auto one = [&](hipStream_t q) -> int {
     op->halt_cur = ir.ctl + wck::kCtlHalt;
-    const int rc2 = inner_iteration<R>(op, N, pd, r, p, mmp, x, aDp, q);
+    const int rc2 = inner_iteration<R>(op, N, pd, r, p, mmp, x, aDp, q, {0, 0.0, ir.dat, ir.ctl, ir.hist});
     op->halt_cur = nullptr;
-    if (rc2) return rc2;
-    wck::iter_check(N, 0, 0.0, st, ir.dat, ir.ctl, ir.hist, q);
-    WC_LAUNCHED();
-    return WC_OK;
+    return rc2;
   };
   const int cap = chunk_cap(op, N, op->chunk);
   std::vector<double> clast(c0);
@@ -447,7 +444,7 @@ static int mixed_impl(wc_operator *hi, wc_operator *lo, int N, int pd, void *dst
   }
   // |src|^2 over both parities (a full field is two half fields back to back)
   wck::dot_partials_rhs<double>(2 * n, N, src, src, hi->partials, nullptr, s);
-  wck::reduce_final_rhs(hi->partials, wck::kRedBlocks, N, sth + 8 * N, s);
+  wck::reduce_final_rhs(hi->partials, wck::red_blocks(2 * n, N), N, sth + 8 * N, s);
   // guess: y = L^-1 dst = A_D dst_D; with a zero guess (all right-hand
   // sides) the first true residual is b_s itself
   site_op<double>(hi, N, pd, 0, half(dst, pd), xh, nullptr, s);
@@ -507,7 +504,7 @@ static int mixed_impl(wc_operator *hi, wc_operator *lo, int N, int pd, void *dst
         if ((rc2 = mpc_impl<double>(hi, N, pd, 0, mp, xh, nullptr, s, aD))) return rc2;
         wck::resid_d2f(n, N, bs, mp, rl, hi->partials, s);
       }
-      wck::reduce_final_rhs(hi->partials, wck::kRedBlocks, N, sth + 9 * N, s);
+      wck::reduce_final_rhs(hi->partials, wck::red_blocks(n, N), N, sth + 9 * N, s);
       if ((rc2 = mpc_impl<float>(lo, N, pd, 1, ml, rl, nullptr, s))) return rc2;
       if ((rc2 = norm2_rhs<float>(lo, N, ml, sth + 10 * N, s))) return rc2;
     } else {
@@ -593,13 +590,11 @@ static int mixed_impl(wc_operator *hi, wc_operator *lo, int N, int pd, void *dst
   const double d2 = delta * delta;
   auto one = [&](hipStream_t q) -> int {
     lo->halt_cur = ir.ctl + wck::kCtlHalt;
-    const int rc2 = lo_single ? inner_iteration<float>(lo, N, pd, rl, pl, ml, xl, aDl, q, nullptr, nullptr, h16)
-                              : inner_iteration<double>(lo, N, pd, rl, pl, ml, xl, aDl, q);
+    const IterCheck chk{1, d2, ir.dat, ir.ctl, ir.hist};
+    const int rc2 = lo_single ? inner_iteration<float>(lo, N, pd, rl, pl, ml, xl, aDl, q, chk, nullptr, nullptr, h16)
+                              : inner_iteration<double>(lo, N, pd, rl, pl, ml, xl, aDl, q, chk);
     lo->halt_cur = nullptr;
-    if (rc2) return rc2;
-    wck::iter_check(N, 1, d2, stl, ir.dat, ir.ctl, ir.hist, q);
-    WC_LAUNCHED();
-    return WC_OK;
+    return rc2;
   };
   std::vector<uintptr_t> key = {1, (uintptr_t)N, (uintptr_t)pd, (uintptr_t)h16, (uintptr_t)rl, (uintptr_t)pl,
                                 (uintptr_t)ml, (uintptr_t)xl, (uintptr_t)aDl, (uintptr_t)stl};

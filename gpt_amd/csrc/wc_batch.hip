@@ -311,7 +311,7 @@ static int batch_reliable(wc_batch *b) {
                           clov_roff(hi));
     if ((rc = mpc_impl<double>(hi, N, b->pd, 0, b->mp, b->xh, nullptr, s, aD, b->partials))) return rc;
     wck::resid_d2f(n, N, b->bs, b->mp, b->rl, b->partials, s);
-    wck::reduce_final_rhs(b->partials, wck::kRedBlocks, N, b->st + 8 * N, s);
+    wck::reduce_final_rhs(b->partials, wck::red_blocks(n, N), N, b->st + 8 * N, s);
     if ((rc = mpc_impl<float>(lo, N, b->pd, 1, b->ml, b->rl, nullptr, s, nullptr, b->partials))) return rc;
     wck::dot_partials_rhs<float>(n, N, b->ml, b->ml, b->partials, nullptr, s);
   } else {
@@ -320,11 +320,11 @@ static int batch_reliable(wc_batch *b) {
     if ((rc = mpc_impl<double>(hi, N, b->pd, 0, b->mp, b->xh, nullptr, s, nullptr, b->partials))) return rc;
     wck::axpy<double>(n, -1.0, 0.0, b->mp, b->bs, b->rs, s);
     wck::dot_partials_rhs<double>(n, N, b->rs, b->rs, b->partials, nullptr, s);
-    wck::reduce_final_rhs(b->partials, wck::kRedBlocks, N, b->st + 8 * N, s);
+    wck::reduce_final_rhs(b->partials, wck::red_blocks(n, N), N, b->st + 8 * N, s);
     if ((rc = mpc_impl<double>(hi, N, b->pd, 1, b->rh, b->rs, nullptr, s, nullptr, b->partials))) return rc;
     wck::dot_partials_rhs<double>(n, N, b->rh, b->rh, b->partials, nullptr, s);
   }
-  wck::reduce_final_rhs(b->partials, wck::kRedBlocks, N, b->st + 9 * N, s);
+  wck::reduce_final_rhs(b->partials, wck::red_blocks(n, N), N, b->st + 9 * N, s);
   WC_LAUNCHED();
   WC_HIP(hipMemcpyAsync(b->host + 8 * N, b->st + 8 * N, sizeof(double) * 2 * N, hipMemcpyDeviceToHost, s));
   WC_HIP(hipStreamSynchronize(s));
@@ -419,7 +419,7 @@ int wc_batch_create(wc_operator *op, wc_operator *inner, int parity, int nslots,
   for (void *&q : b->one) alloc(&q, hbytes(op));
   for (void *&q : b->lone) alloc(&q, hbytes(inner));
   alloc((void **)&b->st, sizeof(double) * 16 * N);
-  alloc((void **)&b->partials, sizeof(double) * std::max(wck::kRedBlocks, wck::hop_blocks(op->g)) * N);
+  alloc((void **)&b->partials, sizeof(double) * 2 * red_partials(op, N));
   if (rc == WC_OK && hipHostMalloc((void **)&b->host, sizeof(double) * 16 * N, hipHostMallocDefault) != hipSuccess) {
     g_err = "wc_batch_create: hipHostMalloc failed";
     rc = WC_ERR_HIP;
@@ -645,16 +645,14 @@ int wc_batch_step(wc_batch *b, int iters, int *finished, int *nfinished) {
   const double d2 = b->delta * b->delta;
   auto one = [&](hipStream_t q) -> int {
     lo->halt_cur = ir.ctl + wck::kCtlHalt;
+    const IterCheck chk{1, d2, ir.dat, ir.ctl, ir.hist};
     const int rc2 = lo->prec == WC_SINGLE
-                        ? inner_iteration<float>(lo, N, b->pd, b->rl, b->pl, b->ml, b->xl, b->aD, q, b->st,
+                        ? inner_iteration<float>(lo, N, b->pd, b->rl, b->pl, b->ml, b->xl, b->aD, q, chk, b->st,
                                                  b->partials, b->h16)
-                        : inner_iteration<double>(lo, N, b->pd, b->rl, b->pl, b->ml, b->xl, b->aD, q, b->st,
+                        : inner_iteration<double>(lo, N, b->pd, b->rl, b->pl, b->ml, b->xl, b->aD, q, chk, b->st,
                                                   b->partials);
     lo->halt_cur = nullptr;
-    if (rc2) return rc2;
-    wck::iter_check(N, 1, d2, b->st, ir.dat, ir.ctl, ir.hist, q);
-    WC_LAUNCHED();
-    return WC_OK;
+    return rc2;
   };
   std::vector<uintptr_t> key = {2, (uintptr_t)N, (uintptr_t)b->pd, (uintptr_t)b->h16, (uintptr_t)b->rl,
                                 (uintptr_t)b->pl, (uintptr_t)b->ml, (uintptr_t)b->xl, (uintptr_t)b->aD,

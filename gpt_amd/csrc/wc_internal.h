@@ -216,10 +216,16 @@ inline int ensure_tmp(wc_operator *op, size_t n, int nrhs, hipStream_t s) {
   return WC_OK;
 }
 
+// per-block partials of one reduction over a half field (or a full one)
+inline size_t red_partials(const wc_operator *op, int nrhs) {
+  return (size_t)std::max(wck::kRedBlocks, wck::hop_blocks(op->g)) * nrhs;
+}
+
 // reduction partials and CG scalars for nrhs right-hand sides (s as for
 // ensure_tmp)
 inline int ensure_red(wc_operator *op, int nrhs, hipStream_t s) {
-  const size_t np = (size_t)std::max(wck::kRedBlocks, wck::hop_blocks(op->g)) * nrhs;
+  // two sets: an iteration's inner products and its residual norms
+  const size_t np = 2 * red_partials(op, nrhs);
   if (np > op->npartials) {
     (void)wc_dev_free_on(op->partials, s);
     op->partials = nullptr;
@@ -522,27 +528,53 @@ inline int norm2_rhs(wc_operator *op, int nrhs, const void *x, double *dev_out, 
   if (rc) return rc;
   const long n = op->g.Vh * 12 * nrhs;
   wck::dot_partials_rhs<R>(n, nrhs, x, x, op->partials, nullptr, s);
-  wck::reduce_final_rhs(op->partials, wck::kRedBlocks, nrhs, dev_out, s);
+  wck::reduce_final_rhs(op->partials, wck::red_blocks(n, nrhs), nrhs, dev_out, s);
   WC_LAUNCHED();
   return WC_OK;
 }
 
+constexpr long kFewPartials = 1024;
+
+// the device test that ends a run of iterations (wck::iter_check)
+struct IterCheck {
+  int mode;
+  double delta2;
+  double *dat;
+  int *ctl;
+  double *hist;
+};
+
 // one iteration of the inner CG on lo: mmp = A p (A_D^-1 p in aD), alpha,
-// r -= alpha mmp, beta, x += alpha p, p = beta p + r, aD = A_D^-1 p
+// r -= alpha mmp, beta, x += alpha p, p = beta p + r, aD = A_D^-1 p; then the
+// test.  partials: 2 * red_partials.  Where the partials are few (1024 in all
+// right-hand sides together: up to 16^3 x 32 for one, 8^4 for 12) alpha is formed
+// inside the r update, and beta together with the test: two launches less,
+// each 4 us when an iteration's kernels are as short (8^4 FP64, one right-hand
+// side: 14 us less an iteration, with the shorter reductions).
 template <typename R>
 inline int inner_iteration(wc_operator *lo, int N, int pd, void *r, void *p, void *mmp, void *x, void *aD,
-                           hipStream_t s, double *st = nullptr, double *partials = nullptr, int half = 0) {
+                           hipStream_t s, const IterCheck &chk, double *st = nullptr, double *partials = nullptr,
+                           int half = 0) {
   int rc;
   const long n = lo->g.Vh * 12 * N;
   if (!st) st = lo->st;
   if (!partials) partials = lo->partials;
+  double *rp = partials + red_partials(lo, N);
   const int *halt = lo->halt_cur;
+  const int nd = wck::hop_blocks(lo->g), nr = wck::red_blocks(n, N);
   if ((rc = mpc_impl<R>(lo, N, pd, 2, mmp, p, p, s, aD, partials, half))) return rc;
-  wck::cg_alpha(partials, wck::hop_blocks(lo->g), N, st, s, halt);
-  wck::cg_update_r<R>(n, N, st, r, mmp, partials, s, halt);
-  wck::cg_beta(partials, wck::kRedBlocks, N, st, s, halt);
+  const bool alpha_in = (long)nd * N <= kFewPartials, check_in = (long)nr * N <= kFewPartials;
+  if (alpha_in) {
+    wck::cg_update_r<R>(n, N, st, r, mmp, rp, s, halt, partials, nd);
+  } else {
+    wck::cg_alpha(partials, nd, N, st, s, halt);
+    wck::cg_update_r<R>(n, N, st, r, mmp, rp, s, halt);
+  }
+  if (check_in) wck::cg_beta_check(rp, nr, N, chk.mode, chk.delta2, st, chk.dat, chk.ctl, chk.hist, s);
+  else wck::cg_beta(rp, nr, N, st, s, halt);
   wck::cg_update_xp<R>(lo->g, N, pd, st, r, p, x, clov_inv(lo, pd), 1.0 / lo->diag, aD,
-                       lo->open_bc ? 1 : 0, s, half, halt, clov_roff(lo));
+                       lo->open_bc ? 1 : 0, s, half, check_in ? chk.ctl + wck::kCtlHaltX : halt, clov_roff(lo));
+  if (!check_in) wck::iter_check(N, chk.mode, chk.delta2, st, chk.dat, chk.ctl, chk.hist, s);
   WC_LAUNCHED();
   return WC_OK;
 }
@@ -589,7 +621,7 @@ inline int pow2_floor(double n, int cap) {
 }
 
 // Runs up to K (a power of two <= 32) iterations: enqueue(q) enqueues one
-// iteration followed by iter_check on stream q (with the operator's halt_cur
+// iteration with its test on stream q (with the operator's halt_cur
 // set to the run's halt word).  K > 1 replays a graph captured once per K and
 // key.  On return (the stream synchronised) hctl and the first
 // hctl[kCtlIter] rows of hhist (nrhs each) hold the run's outcome.
@@ -610,6 +642,7 @@ inline int run_iterations(IterRun &ir, const std::vector<uintptr_t> &key, int K,
   ir.hctl[wck::kCtlMax] = K;
   ir.hctl[wck::kCtlErr] = 0;
   ir.hctl[wck::kCtlTrig] = 0;
+  ir.hctl[wck::kCtlHaltX] = 0;
   WC_HIP(hipMemcpyAsync(ir.ctl, ir.hctl, IterRun::kCtlBytes, hipMemcpyHostToDevice, s));
   if (K <= 1) {
     if ((rc = enqueue(s))) return rc;

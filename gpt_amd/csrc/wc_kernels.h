@@ -119,12 +119,13 @@ void site_clover(const Geom &g, int nrhs, int p, const void *blocks, double diag
                  const void *y, int open_bc, hipStream_t s, int half = 0, const long *roff = nullptr);
 
 // Per-right-hand-side reductions over fields whose innermost index is the
-// RHS (nrhs of them): partials[r * kRedBlocks + b] for b < kRedBlocks, then
+// RHS (nrhs of them): partials[r * nb + b] for b < nb = red_blocks(n, nrhs), then
 // out[r] = sum over b in fixed order.
 template <typename R>
 void dot_partials_rhs(long n, int nrhs, const void *a, const void *b, double *pre, double *pim, hipStream_t s);
 void reduce_final_rhs(const double *partials, int nblocks, int nrhs, double *out, hipStream_t s);
 int rhs_block_threads(int nrhs);
+int red_blocks(long n, int nrhs);  // at most kRedBlocks
 // hi[e] += (double) lo[e] (FP32 -> FP64 accumulation of n entries)
 void accumulate_f2d(long n, const void *lo, void *hi, hipStream_t s);
 // x = 0 for n complex entries of R (a kernel, so it can sit in a captured graph)
@@ -185,10 +186,12 @@ void build_clover(const Geom &g, const void *Unat, const CloverParams &cp, void 
 // word; while it is non-zero the launch does nothing.
 void cg_alpha(const double *partials, int nblocks, int nrhs, double *st, hipStream_t s, const int *halt = nullptr);
 void cg_beta(const double *partials, int nblocks, int nrhs, double *st, hipStream_t s, const int *halt = nullptr);
-// r -= alpha_r mmp with per-RHS partials of |r|^2 (kRedBlocks blocks)
+// r -= alpha_r mmp with per-RHS partials of |r|^2 (red_blocks(n, nrhs) blocks);
+// dp (optional): the ndp partials of <p, A p>, from which it forms d and alpha
+// itself (then no cg_alpha; partials must not overlap dp)
 template <typename R>
-void cg_update_r(long n, int nrhs, const double *st, void *r, const void *mmp, double *partials, hipStream_t s,
-                 const int *halt = nullptr);
+void cg_update_r(long n, int nrhs, double *st, void *r, const void *mmp, double *partials, hipStream_t s,
+                 const int *halt = nullptr, const double *dp = nullptr, int ndp = 0);
 // x += alpha_r p ; p = beta_r p + r ; t = A p with A the clover-inverse
 // blocks of parity par (or diag when null), zero on an open boundary.
 // half: FP32 only, p and t stored as 16-bit (kS16Half / kS16Bf16).
@@ -209,6 +212,7 @@ enum {
   kCtlMax = 2,    // iterations allowed in this run
   kCtlErr = 3,    // 1 + first right-hand side with a non-finite |r|^2, or 0
   kCtlTrig = 4,   // mode 1: a reliable update is due
+  kCtlHaltX = 5,  // cg_beta_check: set one iteration after kCtlHalt (the x/p update's halt word)
   kCtlInts = 16,  // ints of the control block (64 B)
 };
 // dat rows (kMaxRhs entries each): 0 stop limit (mode 0: eps^2 |b|^2;
@@ -227,6 +231,10 @@ constexpr int kMaxChunk = 64;  // iterations per run (rows of hist)
 // non-finite |r|^2 halts with kCtlErr; iteration kCtlMax halts.
 void iter_check(int nrhs, int mode, double delta2, double *st, double *dat, int *ctl, double *hist,
                 hipStream_t s);
+// cg_beta and iter_check in one launch, before cg_update_xp (whose halt word
+// is then ctl + kCtlHaltX)
+void cg_beta_check(const double *partials, int nblocks, int nrhs, int mode, double delta2, double *st, double *dat,
+                   int *ctl, double *hist, hipStream_t s);
 
 // per-right-hand-side scalings of the 16-bit-storage inner solve (n complex
 // entries, RHS innermost): dst = (float) (src * f[r]); x16 *= f[r];

@@ -4,6 +4,8 @@
 // conversions and the link / clover set-up.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "wc_kernels.h"
 #include "wc_site.h"
 
@@ -599,12 +601,25 @@ template void build_clover<float>(const Geom &, const void *, const CloverParams
 // block size: the largest multiple of nrhs not above 256, so that a thread's
 // elements (strided by a multiple of nrhs) all belong to one RHS
 int rhs_block_threads(int nrhs) { return (256 / nrhs) * nrhs; }
+// blocks of the per-RHS reductions over n entries: no more than have entries
+// (with 1024 for the 24576 entries of an 8^4 half field, nine of ten idle and
+// the sum over their partials as long as ever)
+int red_blocks(long n, int nrhs) {
+  const long t = rhs_block_threads(nrhs);
+  return (int)std::min<long>(kRedBlocks, std::max<long>(1, (n + t - 1) / t));
+}
 
-// sum of lds[0..nt) over the entries of RHS threadIdx.x (< nrhs), fixed order
-__device__ __forceinline__ double seg_sum(const double *lds, int nt, int nrhs) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < nt; i += nrhs) s += lds[i];
-  return s;
+// lds[r] = sum over the entries of RHS r (< nrhs) among lds[0..nt), by halves
+// in a fixed order (one thread adding up the 256 entries of a single RHS took
+// 8 us); every thread of the block calls it, nt a multiple of nrhs
+__device__ __forceinline__ void seg_sum(double *lds, int nt, int nrhs) {
+  __syncthreads();
+  for (int m = nt / nrhs; m > 1;) {
+    const int h = (m + 1) >> 1;
+    if ((int)threadIdx.x < (m - h) * nrhs) lds[threadIdx.x] += lds[threadIdx.x + h * nrhs];
+    __syncthreads();
+    m = h;
+  }
 }
 
 template <typename R>
@@ -619,17 +634,18 @@ __global__ __launch_bounds__(256) void k_dot_rhs(long n, int N, const typename c
     si += ax * by - ay * bx;
   }
   lr[threadIdx.x] = sr;
-  li[threadIdx.x] = si;
-  __syncthreads();
-  if ((int)threadIdx.x < N) {
-    pre[(long)threadIdx.x * gridDim.x + blockIdx.x] = seg_sum(lr, blockDim.x, N);
-    if (pim) pim[(long)threadIdx.x * gridDim.x + blockIdx.x] = seg_sum(li, blockDim.x, N);
+  seg_sum(lr, blockDim.x, N);
+  if ((int)threadIdx.x < N) pre[(long)threadIdx.x * gridDim.x + blockIdx.x] = lr[threadIdx.x];
+  if (pim) {
+    li[threadIdx.x] = si;
+    seg_sum(li, blockDim.x, N);
+    if ((int)threadIdx.x < N) pim[(long)threadIdx.x * gridDim.x + blockIdx.x] = li[threadIdx.x];
   }
 }
 template <typename R>
 void dot_partials_rhs(long n, int nrhs, const void *a, const void *b, double *pre, double *pim, hipStream_t s) {
   using C = typename c2<R>::t;
-  k_dot_rhs<R><<<kRedBlocks, rhs_block_threads(nrhs), 0, s>>>(n, nrhs, (const C *)a, (const C *)b, pre, pim);
+  k_dot_rhs<R><<<red_blocks(n, nrhs), rhs_block_threads(nrhs), 0, s>>>(n, nrhs, (const C *)a, (const C *)b, pre, pim);
 }
 template void dot_partials_rhs<double>(long, int, const void *, const void *, double *, double *, hipStream_t);
 template void dot_partials_rhs<float>(long, int, const void *, const void *, double *, double *, hipStream_t);
@@ -767,17 +783,50 @@ void cg_beta(const double *partials, int nblocks, int nrhs, double *st, hipStrea
   k_cg_beta<<<nrhs, 256, 0, s>>>(partials, nblocks, nrhs, st, halt);
 }
 
-// r -= alpha_r mmp; partial |r|^2 per RHS
-template <typename R>
-__global__ __launch_bounds__(256) void k_cg_update_r(long n, int N, const double *st, typename c2<R>::t *r,
+// sum of p[r * nb + b] over b by one whole wave, in a fixed order
+__device__ __forceinline__ double wave_total(const double *p, int nb, int r) {
+  const double *q = p + (long)r * nb;
+  double s = 0.0;
+  for (int b = threadIdx.x & 63; b < nb; b += 64) s += q[b];
+  return wave_sum(s);
+}
+
+// r -= alpha_r mmp; partial |r|^2 per RHS.  ALPHA: every block first forms
+// d_r (row 1) and alpha_r (row 2) from the ndp partials dp of <p, A p> itself,
+// its waves taking the right-hand sides in turn, and block 0 stores them: the
+// launch of k_cg_alpha and its wait saved (4 us of an iteration), for a read
+// of the partials per block
+template <typename R, bool ALPHA>
+__global__ __launch_bounds__(256) void k_cg_update_r(long n, int N, double *st, typename c2<R>::t *r,
                                                      const typename c2<R>::t *mmp, double *pre,
-                                                     const int *halt) {
+                                                     const int *halt, const double *dp, int ndp) {
   using C = typename c2<R>::t;
   if (halt && *halt) return;
   __shared__ double lds[256];
   const long stride = (long)gridDim.x * blockDim.x;
   const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const R a = (R)st[2 * N + (int)(i0 % N)];
+  const int rr = (int)(i0 % N);
+  R a;
+  if constexpr (ALPHA) {
+    __shared__ double al[kMaxRhs];
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;  // whole waves only
+    if (w < nw)
+      for (int k = w; k < N; k += nw) {
+        const double d = wave_total(dp, ndp, k);
+        if ((threadIdx.x & 63) == 0) {
+          const double v = (st[5 * N + k] != 0.0 && d != 0.0) ? st[0 * N + k] / d : 0.0;
+          al[k] = v;
+          if (blockIdx.x == 0) {
+            st[1 * N + k] = d;
+            st[2 * N + k] = v;
+          }
+        }
+      }
+    __syncthreads();
+    a = (R)al[rr];
+  } else {
+    a = (R)st[2 * N + rr];
+  }
   double s = 0.0;
   for (long i = i0; i < n; i += stride) {
     C rv = r[i];
@@ -787,20 +836,23 @@ __global__ __launch_bounds__(256) void k_cg_update_r(long n, int N, const double
     s += (double)rv.x * (double)rv.x + (double)rv.y * (double)rv.y;
   }
   lds[threadIdx.x] = s;
-  __syncthreads();
-  if ((int)threadIdx.x < N) pre[(long)threadIdx.x * gridDim.x + blockIdx.x] = seg_sum(lds, blockDim.x, N);
+  seg_sum(lds, blockDim.x, N);
+  if ((int)threadIdx.x < N) pre[(long)threadIdx.x * gridDim.x + blockIdx.x] = lds[threadIdx.x];
 }
 template <typename R>
-void cg_update_r(long n, int nrhs, const double *st, void *r, const void *mmp, double *partials, hipStream_t s,
-                 const int *halt) {
+void cg_update_r(long n, int nrhs, double *st, void *r, const void *mmp, double *partials, hipStream_t s,
+                 const int *halt, const double *dp, int ndp) {
   using C = typename c2<R>::t;
-  k_cg_update_r<R><<<kRedBlocks, rhs_block_threads(nrhs), 0, s>>>(n, nrhs, st, (C *)r, (const C *)mmp, partials,
-                                                                  halt);
+  const int nb = red_blocks(n, nrhs), nt = rhs_block_threads(nrhs);
+  if (dp)
+    k_cg_update_r<R, true><<<nb, nt, 0, s>>>(n, nrhs, st, (C *)r, (const C *)mmp, partials, halt, dp, ndp);
+  else
+    k_cg_update_r<R, false><<<nb, nt, 0, s>>>(n, nrhs, st, (C *)r, (const C *)mmp, partials, halt, nullptr, 0);
 }
-template void cg_update_r<double>(long, int, const double *, void *, const void *, double *, hipStream_t,
-                                  const int *);
-template void cg_update_r<float>(long, int, const double *, void *, const void *, double *, hipStream_t,
-                                 const int *);
+template void cg_update_r<double>(long, int, double *, void *, const void *, double *, hipStream_t, const int *,
+                                  const double *, int);
+template void cg_update_r<float>(long, int, double *, void *, const void *, double *, hipStream_t, const int *,
+                                 const double *, int);
 
 // x += alpha_r p ; p = beta_r p + r ; t = A p (site-local, parity par: the
 // clover inverse blocks A, or diag when A is null; zero on an open boundary).
@@ -901,10 +953,9 @@ template void cg_update_xp<double>(const Geom &, int, int, const double *, const
 template void cg_update_xp<float>(const Geom &, int, int, const double *, const void *, void *, void *,
                                   const void *, double, void *, int, hipStream_t, int, const int *, const long *);
 
-// one wave; lane r handles right-hand side r (nrhs <= 64)
-__global__ __launch_bounds__(64) void k_iter_check(int N, int mode, double delta2, double *st, double *dat,
-                                                   int *ctl, double *hist) {
-  if (ctl[kCtlHalt]) return;
+// one wave; lane r handles right-hand side r (nrhs <= 64), cp: its |r|^2
+__device__ __forceinline__ void iter_check_lane(int N, int mode, double delta2, double cp, double *st, double *dat,
+                                                int *ctl, double *hist) {
   const int r = threadIdx.x;
   const int k = ctl[kCtlIter];
   if (k >= kMaxChunk) {  // the history holds kMaxChunk iterations
@@ -914,7 +965,6 @@ __global__ __launch_bounds__(64) void k_iter_check(int N, int mode, double delta
   const bool act = r < N && st[5 * N + r] != 0.0;
   bool bad = false, trig = false, left = false;
   if (act) {
-    const double cp = st[4 * N + r];
     hist[(long)k * N + r] = cp;
     bad = !isfinite(cp);
     if (mode == 0) {
@@ -939,6 +989,45 @@ __global__ __launch_bounds__(64) void k_iter_check(int N, int mode, double delta
     if (trigm) ctl[kCtlTrig] = 1;
     if (badm || trigm || !leftm || k + 1 >= ctl[kCtlMax]) ctl[kCtlHalt] = 1;
   }
+}
+__global__ __launch_bounds__(64) void k_iter_check(int N, int mode, double delta2, double *st, double *dat,
+                                                   int *ctl, double *hist) {
+  if (ctl[kCtlHalt]) return;
+  const int r = threadIdx.x;
+  iter_check_lane(N, mode, delta2, r < N ? st[4 * N + r] : 0.0, st, dat, ctl, hist);
+}
+
+// k_cg_beta of every right-hand side, then k_iter_check, in one workgroup: a
+// launch and its wait saved where the partials are few.  It runs before the
+// iteration's k_cg_update_xp, which therefore looks at kCtlHaltX: set here by
+// the first iteration after the one that halted the run.
+__global__ __launch_bounds__(256) void k_cg_beta_check(const double *p, int nb, int N, int mode, double delta2,
+                                                       double *st, double *dat, int *ctl, double *hist) {
+  __shared__ double cp[kMaxRhs];
+  if (ctl[kCtlHalt]) {
+    if (threadIdx.x == 0) ctl[kCtlHaltX] = 1;
+    return;
+  }
+  for (int r = threadIdx.x >> 6; r < N; r += 4) {
+    const double s = wave_total(p, nb, r);
+    if ((threadIdx.x & 63) == 0) {
+      cp[r] = s;
+      st[4 * N + r] = s;
+      if (st[5 * N + r] != 0.0) {
+        st[3 * N + r] = s / st[0 * N + r];
+        st[0 * N + r] = s;
+      } else {
+        st[3 * N + r] = 0.0;
+      }
+    }
+  }
+  __syncthreads();  // also: every wave has read kCtlHalt
+  if (threadIdx.x < 64)
+    iter_check_lane(N, mode, delta2, (int)threadIdx.x < N ? cp[threadIdx.x] : 0.0, st, dat, ctl, hist);
+}
+void cg_beta_check(const double *partials, int nblocks, int nrhs, int mode, double delta2, double *st, double *dat,
+                   int *ctl, double *hist, hipStream_t s) {
+  k_cg_beta_check<<<1, 256, 0, s>>>(partials, nblocks, nrhs, mode, delta2, st, dat, ctl, hist);
 }
 void iter_check(int nrhs, int mode, double delta2, double *st, double *dat, int *ctl, double *hist,
                 hipStream_t s) {
@@ -997,11 +1086,11 @@ __global__ __launch_bounds__(256) void k_resid_d2f(long n, int N, const double2 
     sr += v.x * v.x + v.y * v.y;
   }
   lr[threadIdx.x] = sr;
-  __syncthreads();
-  if ((int)threadIdx.x < N) pre[(long)threadIdx.x * gridDim.x + blockIdx.x] = seg_sum(lr, blockDim.x, N);
+  seg_sum(lr, blockDim.x, N);
+  if ((int)threadIdx.x < N) pre[(long)threadIdx.x * gridDim.x + blockIdx.x] = lr[threadIdx.x];
 }
 void resid_d2f(long n, int nrhs, const void *bs, const void *mp, void *rl, double *partials, hipStream_t s) {
-  k_resid_d2f<<<kRedBlocks, rhs_block_threads(nrhs), 0, s>>>(n, nrhs, (const double2 *)bs, (const double2 *)mp,
+  k_resid_d2f<<<red_blocks(n, nrhs), rhs_block_threads(nrhs), 0, s>>>(n, nrhs, (const double2 *)bs, (const double2 *)mp,
                                                              (float2 *)rl, partials);
 }
 

@@ -48,6 +48,7 @@ _I, _L, _D = ctypes.c_int, ctypes.c_long, ctypes.c_double
 SIGNATURES = {
     "wc_create": (_I, [ctypes.POINTER(wc_params), _P, _P, ctypes.POINTER(_P)]),
     "wc_update": (_I, [_P, _P, _P]),
+    "wc_update_links": (_I, [_P, _P, _P, _P, _P, _P]),
     "wc_set_mass": (_I, [_P, _D, _P]),
     "wc_destroy": (_I, [_P]),
     "wc_half_volume": (_L, [_P]),

@@ -81,9 +81,9 @@ int build_mass_blocks(const wc_operator *op, double mass, void *ai0, void *ai1, 
   cp.diag = mass + 1.0 + 3.0 * op->p.nu / op->p.xi_0;  // 1/(2 kappa), as set_mass_values
   WC_HIP(hipMemsetAsync(err, 0, sizeof(int), s));
   if (op->prec == WC_DOUBLE)
-    wck::build_clover<double>(op->g, op->Unat, cp, a0, a1, ai0, ai1, err, s);
+    wck::build_clover<double>(op->g, op->G, cp, a0, a1, ai0, ai1, err, s);
   else
-    wck::build_clover<float>(op->g, op->Unat, cp, a0, a1, ai0, ai1, err, s);
+    wck::build_clover<float>(op->g, op->G, cp, a0, a1, ai0, ai1, err, s);
   WC_LAUNCHED();
   int herr = 0;
   WC_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -92,28 +92,61 @@ int build_mass_blocks(const wc_operator *op, double mass, void *ai0, void *ai1, 
   return WC_OK;
 }
 
-static int build_all(wc_operator *op, hipStream_t s) {
-  const Geom &g = op->g;
+// the clover blocks and their inverses from the kept gauge field
+static int build_own_clover(wc_operator *op, hipStream_t s) {
+  if (!op->has_clover) return WC_OK;
+  WC_HIP(hipMemsetAsync(op->err, 0, sizeof(int), s));
+  wck::CloverParams cp = clover_params(op);
   if (op->prec == WC_DOUBLE)
-    wck::build_links<double>(g, op->Unat, op->nl, op->W[0], op->W[1], s);
+    wck::build_clover<double>(op->g, op->G, cp, op->A[0], op->A[1], op->Ai[0], op->Ai[1], op->err, s);
   else
-    wck::build_links<float>(g, op->Unat, op->nl, op->W[0], op->W[1], s);
+    wck::build_clover<float>(op->g, op->G, cp, op->A[0], op->A[1], op->Ai[0], op->Ai[1], op->err, s);
   WC_LAUNCHED();
-  if (op->has_clover) {
-    WC_HIP(hipMemsetAsync(op->err, 0, sizeof(int), s));
-    wck::CloverParams cp = clover_params(op);
-    if (op->prec == WC_DOUBLE)
-      wck::build_clover<double>(g, op->Unat, cp, op->A[0], op->A[1], op->Ai[0], op->Ai[1], op->err, s);
-    else
-      wck::build_clover<float>(g, op->Unat, cp, op->A[0], op->A[1], op->Ai[0], op->Ai[1], op->err, s);
-    WC_LAUNCHED();
-    int herr = 0;
-    WC_HIP(hipMemcpyAsync(&herr, op->err, sizeof(int), hipMemcpyDeviceToHost, s));
-    WC_HIP(hipStreamSynchronize(s));
-    if (herr) WC_FAIL(WC_ERR_NUMERIC, "clover block is singular or near-singular at some site (mass %g)", op->mass);
-  }
+  int herr = 0;
+  WC_HIP(hipMemcpyAsync(&herr, op->err, sizeof(int), hipMemcpyDeviceToHost, s));
+  WC_HIP(hipStreamSynchronize(s));
+  if (herr) WC_FAIL(WC_ERR_NUMERIC, "clover block is singular or near-singular at some site (mass %g)", op->mass);
   return WC_OK;
 }
+
+// whether a kernel can read p: device (or managed) memory
+static bool on_device(const void *p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // host memory that HIP does not know
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
+}
+
+// links and clover from four natural link fields; one that a kernel cannot
+// read as it is (host memory, an odd multiple of 8 bytes) is first copied to
+// its place in the kept field
+static int build_all(wc_operator *op, const void *const U[4], hipStream_t s) {
+  const size_t bytes = (size_t)op->g.V * 9 * 16;
+  const void *dev[4];
+  for (int mu = 0; mu < 4; ++mu) {
+    dev[mu] = U[mu];
+    if (((uintptr_t)U[mu] & 15) == 0 && on_device(U[mu])) continue;
+    void *own = (char *)op->G + mu * bytes;
+    WC_HIP(hipMemcpyAsync(own, U[mu], bytes, hipMemcpyDefault, s));
+    dev[mu] = own;
+  }
+  if (op->prec == WC_DOUBLE)
+    wck::gauge_setup<double>(op->g, dev, op->nl, op->G, op->W[0], op->W[1], s);
+  else
+    wck::gauge_setup<float>(op->g, dev, op->nl, op->G, op->W[0], op->W[1], s);
+  WC_LAUNCHED();
+  return build_own_clover(op, s);
+}
+
+// the four directions of a field [4][V][3][3]
+struct FourLinks {
+  const void *U[4];
+  FourLinks(const wc_operator *op, const void *u) {
+    for (int mu = 0; mu < 4; ++mu) U[mu] = (const char *)u + (size_t)mu * op->g.V * 9 * 16;
+  }
+};
 
 static void set_mass_values(wc_operator *op, double mass) {
   op->mass = mass;
@@ -181,18 +214,14 @@ int wc_create(const wc_params *p, const void *U, void *stream, wc_operator **out
       chk(wc_dev_malloc(&op->Ai[q], Vh * 36 * op->csz), "wc_dev_malloc(clover inverse)");
     }
   }
-  chk(wc_dev_malloc(&op->Unat, (size_t)op->g.V * 4 * 9 * 16), "wc_dev_malloc(gauge copy)");
+  chk(wc_dev_malloc(&op->G, (size_t)op->g.V * 4 * 9 * 16), "wc_dev_malloc(gauge copy)");
   chk(wc_dev_malloc((void **)&op->err, sizeof(int)), "wc_dev_malloc(flag)");
   if (rc == WC_OK && ensure_red(op, 1, (hipStream_t)stream) != WC_OK) rc = WC_ERR_HIP;
   if (rc != WC_OK) {
     free_op(op);
     return rc;
   }
-  if (hipMemcpyAsync(op->Unat, U, (size_t)op->g.V * 4 * 9 * 16, hipMemcpyDefault, s) != hipSuccess) {
-    free_op(op);
-    WC_FAIL(WC_ERR_HIP, "wc_create: copying the gauge field failed");
-  }
-  rc = build_all(op, s);
+  rc = build_all(op, FourLinks(op, U).U, s);
   if (rc != WC_OK) {
     std::string keep = g_err;
     free_op(op);
@@ -205,16 +234,19 @@ int wc_create(const wc_params *p, const void *U, void *stream, wc_operator **out
 
 int wc_update(wc_operator *op, const void *U, void *stream) {
   if (!op || !U) WC_FAIL(WC_ERR_ARG, "wc_update: null argument");
-  hipStream_t s = (hipStream_t)stream;
-  WC_HIP(hipMemcpyAsync(op->Unat, U, (size_t)op->g.V * 4 * 9 * 16, hipMemcpyDefault, s));
-  return build_all(op, s);
+  return build_all(op, FourLinks(op, U).U, (hipStream_t)stream);
+}
+
+int wc_update_links(wc_operator *op, const void *U0, const void *U1, const void *U2, const void *U3, void *stream) {
+  if (!op || !U0 || !U1 || !U2 || !U3) WC_FAIL(WC_ERR_ARG, "wc_update_links: null argument");
+  const void *const U[4] = {U0, U1, U2, U3};
+  return build_all(op, U, (hipStream_t)stream);
 }
 
 int wc_set_mass(wc_operator *op, double mass, void *stream) {
   if (!op) WC_FAIL(WC_ERR_ARG, "wc_set_mass: null operator");
   set_mass_values(op, mass);
-  if (!op->has_clover) return WC_OK;
-  return build_all(op, (hipStream_t)stream);
+  return build_own_clover(op, (hipStream_t)stream);
 }
 
 int wc_destroy(wc_operator *op) {

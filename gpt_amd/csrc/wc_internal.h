@@ -144,7 +144,7 @@ struct wc_operator {
   void *W[2] = {nullptr, nullptr};
   void *A[2] = {nullptr, nullptr};
   void *Ai[2] = {nullptr, nullptr};
-  void *Unat = nullptr;  // FP64 links [4][V][9], kept to rebuild the clover on set_mass
+  void *G = nullptr;     // FP64 links by parity (gauge_at), kept to rebuild the clover on set_mass
   int *err = nullptr;    // device flag of the clover build
   std::vector<void *> tmp;      // half-field scratch, tmp_bytes each
   size_t tmp_bytes = 0;
@@ -263,7 +263,7 @@ inline void free_op(wc_operator *op) {
     (void)wc_dev_free_idle(op->A[p]);
     (void)wc_dev_free_idle(op->Ai[p]);
   }
-  (void)wc_dev_free_idle(op->Unat);
+  (void)wc_dev_free_idle(op->G);
   (void)wc_dev_free_idle(op->err);
   for (void *q : op->tmp) (void)wc_dev_free_idle(q);
   (void)wc_dev_free_idle(op->partials);

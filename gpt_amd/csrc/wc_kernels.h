@@ -161,9 +161,11 @@ void convert_f2d(long n, const void *src, void *dst, hipStream_t s);
 template <typename R> void import_field(const Geom &g, const void *nat, void *eo, hipStream_t s);
 template <typename R> void export_field(const Geom &g, const void *eo, void *nat, hipStream_t s);
 
-// operator set-up from natural FP64 links Unat[4][V][9]
+// operator set-up from natural FP64 links [V][9], one device pointer a
+// direction: the kept gauge field G (FP64, 36 V complex, blocked by parity) and
+// the hop's links
 template <typename R>
-void build_links(const Geom &g, const void *Unat, int nl, void *W0, void *W1, hipStream_t s);
+void gauge_setup(const Geom &g, const void *const U[4], int nl, void *G, void *W0, void *W1, hipStream_t s);
 
 struct CloverParams {
   double coef[6];          // -csw_{mu nu}/2 for the planes (01,02,03,12,13,23)
@@ -173,11 +175,11 @@ struct CloverParams {
   double cF;
   int open_bc;
 };
-// writes packed A and A^-1 per parity; err_flag (device int) gets 1 on a
-// near-singular block
+// from the kept gauge field, writes packed A and A^-1 per parity; err_flag
+// (device int) gets 1 on a near-singular block
 template <typename R>
 // A0 / A1 may be null (only the inverse wanted)
-void build_clover(const Geom &g, const void *Unat, const CloverParams &cp, void *A0, void *A1,
+void build_clover(const Geom &g, const void *G, const CloverParams &cp, void *A0, void *A1,
                   void *Ai0, void *Ai1, int *err_flag, hipStream_t s);
 
 // CG on nrhs independent right-hand sides with device scalars:

@@ -329,268 +329,345 @@ template void export_field<double>(const Geom &, const void *, void *, hipStream
 template void export_field<float>(const Geom &, const void *, void *, hipStream_t);
 
 // ----------------------------------------------------------- link set-up
-__device__ __forceinline__ long nat_index(const Geom &g, int x, int y, int z, int t) {
-  return (((long)t * g.L[2] + z) * g.L[1] + y) * g.L[0] + x;
+// The gauge field as the set-up kernels keep it: FP64 links in blocks of 64
+// half-sites, the two parities of a block (the 128 natural sites 128 b ..
+// 128 b + 127) one after the other, entry e of U_mu(h, p) at gauge_at + 64 e
+__device__ __forceinline__ const double2 *gauge_at(const double2 *G, const Geom &g, int mu, int p, long h) {
+  return G + (((long)mu * (g.Vh / kBlk) + h / kBlk) * 2 + p) * (9 * kBlk) + h % kBlk;
 }
 
+// Natural links [V][9], one pointer a direction, to the kept gauge field (G)
+// and to the hop's links (W0, W1) in one pass: a workgroup takes 128
+// consecutive natural sites, which are the 64 half-sites 64 b .. 64 b + 63 of
+// both parities.  Each direction's 18 KB are read contiguously into LDS and
+// written from there in the blocked layouts: to G and the forward link of the
+// site itself, and, conjugated, to the backward link of the site x + mu.  A
+// block of G lies where its natural sites lie in U, so that U may be G itself.
+// Bound by HBM: 382 MB read and 1.15 GB written for 24^3 x 48 FP64 take 285 us
+// (5.4 TB/s); reading 144-byte sites lane by lane, the links alone took 834 us,
+// after a copy of the field (73 us).
 template <typename R>
-__global__ void k_build_links(Geom g, const double2 *U, int nl, typename c2<R>::t *W0, typename c2<R>::t *W1) {
+__global__ __launch_bounds__(256) void k_gauge_setup(Geom g, const double2 *U0, const double2 *U1, const double2 *U2,
+                                                     const double2 *U3, int nl, double2 *G, typename c2<R>::t *W0,
+                                                     typename c2<R>::t *W1) {
   using C = typename c2<R>::t;
-  long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= 2 * g.Vh) return;
-  const int p = (int)(i / g.Vh);
-  const long h = i - (long)p * g.Vh;
-  C *W = p ? W1 : W0;
+  __shared__ double2 lds[128 * 9];
+  const int tid = threadIdx.x, hl = tid & 63, p = (tid >> 6) & 1, back = tid >> 7;
+  const long blk = blockIdx.x, h = blk * kBlk + hl;
   int c[4];
   half_coords(g, h, p, c);
-  const long xi = nat_index(g, c[0], c[1], c[2], c[3]);
+  const double2 *mine = lds + 9 * (2 * hl + (c[0] & 1));
+#pragma unroll 1
   for (int mu = 0; mu < 4; ++mu) {
-    int m[4] = {c[0], c[1], c[2], c[3]};
-    m[mu] = (c[mu] + g.L[mu] - 1) % g.L[mu];
-    const long xm = nat_index(g, m[0], m[1], m[2], m[3]);
-    const double2 *uf = U + ((long)mu * g.V + xi) * 9;
-    const double2 *ub = U + ((long)mu * g.V + xm) * 9;
-    for (int e = 0; e < nl; ++e) {
-      const int r = e / 3, col = e % 3;
-      double2 f = uf[e];
-      double2 b = ub[col * 3 + r];  // (U^dag)_{r col} = conj(U_{col r})
-      W[aidx(2 * mu * nl + e, h, 8 * nl)] = cmk<C>((R)f.x, (R)f.y);
-      W[aidx((2 * mu + 1) * nl + e, h, 8 * nl)] = cmk<C>((R)b.x, (R)(-b.y));
+    const double2 *U = (mu == 0 ? U0 : mu == 1 ? U1 : mu == 2 ? U2 : U3) + blk * (128 * 9);
+    __syncthreads();
+    for (int i = tid; i < 128 * 9; i += 256) lds[i] = U[i];
+    __syncthreads();
+    double2 u[9];
+#pragma unroll
+    for (int e = 0; e < 9; ++e) u[e] = mine[e];
+    if (!back) {
+      double2 *o = const_cast<double2 *>(gauge_at(G, g, mu, p, h));
+#pragma unroll
+      for (int e = 0; e < 9; ++e) o[e * kBlk] = u[e];
+      C *w = (p ? W1 : W0) + aidx(2 * mu * nl, h, 8 * nl);
+#pragma unroll
+      for (int e = 0; e < 9; ++e)
+        if (e < nl) w[e * kBlk] = cmk<C>((R)u[e].x, (R)u[e].y);
+    } else {
+      int x[4] = {c[0], c[1], c[2], c[3]};
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (m == mu) x[m] = c[m] == g.L[m] - 1 ? 0 : c[m] + 1;
+      const long hn = half_index(g, x[0], x[1], x[2], x[3]);
+      C *w = (p ? W0 : W1) + aidx((2 * mu + 1) * nl, hn, 8 * nl);
+#pragma unroll
+      for (int e = 0; e < 9; ++e)
+        if (e < nl) {
+          const double2 v = u[(e % 3) * 3 + e / 3];  // (U^dag)_{r col} = conj(U_{col r})
+          w[e * kBlk] = cmk<C>((R)v.x, (R)(-v.y));
+        }
     }
   }
 }
 template <typename R>
-void build_links(const Geom &g, const void *Unat, int nl, void *W0, void *W1, hipStream_t s) {
+void gauge_setup(const Geom &g, const void *const U[4], int nl, void *G, void *W0, void *W1, hipStream_t s) {
   using C = typename c2<R>::t;
-  k_build_links<R><<<elem_blocks(2 * g.Vh), 256, 0, s>>>(g, (const double2 *)Unat, nl, (C *)W0, (C *)W1);
+  k_gauge_setup<R><<<(unsigned)(g.Vh / kBlk), 256, 0, s>>>(g, (const double2 *)U[0], (const double2 *)U[1],
+                                                          (const double2 *)U[2], (const double2 *)U[3], nl,
+                                                          (double2 *)G, (C *)W0, (C *)W1);
 }
-template void build_links<double>(const Geom &, const void *, int, void *, void *, hipStream_t);
-template void build_links<float>(const Geom &, const void *, int, void *, void *, hipStream_t);
+template void gauge_setup<double>(const Geom &, const void *const[4], int, void *, void *, void *, hipStream_t);
+template void gauge_setup<float>(const Geom &, const void *const[4], int, void *, void *, void *, hipStream_t);
 
 // ---------------------------------------------------------- clover set-up
 struct M3 {
   double2 e[9];
 };
-__device__ __forceinline__ M3 ld3(const double2 *U, const Geom &g, int mu, const int x[4]) {
+__device__ __forceinline__ M3 ld3(const double2 *G, const Geom &g, int mu, const int x[4]) {
   M3 m;
-  const long xi = nat_index(g, x[0], x[1], x[2], x[3]);
-  const double2 *p = U + ((long)mu * g.V + xi) * 9;
+  const double2 *p = gauge_at(G, g, mu, (x[0] + x[1] + x[2] + x[3]) & 1, half_index(g, x[0], x[1], x[2], x[3]));
 #pragma unroll
-  for (int k = 0; k < 9; ++k) m.e[k] = p[k];
+  for (int k = 0; k < 9; ++k) m.e[k] = p[k * kBlk];
   return m;
 }
-// op: 0 = A B, 1 = A B^dag, 2 = A^dag B
-__device__ __forceinline__ M3 mm(const M3 &A, const M3 &B, int op) {
+__device__ __forceinline__ M3 dag(const M3 &A) {
+  M3 r;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) r.e[k] = cconj(A.e[(k % 3) * 3 + k / 3]);
+  return r;
+}
+__device__ __forceinline__ M3 neg(const M3 &A) {
+  M3 r;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) r.e[k] = make_double2(-A.e[k].x, -A.e[k].y);
+  return r;
+}
+// A B, or C + A B
+__device__ __forceinline__ M3 mm(const M3 &A, const M3 &B) {
   M3 r;
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      double2 s = make_double2(0.0, 0.0);
+      double2 s = cmul(A.e[i * 3], B.e[j]);
+      s = cmadd(s, A.e[i * 3 + 1], B.e[3 + j]);
+      r.e[i * 3 + j] = cmadd(s, A.e[i * 3 + 2], B.e[6 + j]);
+    }
+  return r;
+}
+__device__ __forceinline__ M3 mma(const M3 &C, const M3 &A, const M3 &B) {
+  M3 r;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double2 a = (op == 2) ? cconj(A.e[k * 3 + i]) : A.e[i * 3 + k];
-        double2 b = (op == 1) ? cconj(B.e[j * 3 + k]) : B.e[k * 3 + j];
-        s = cadd(s, cmul(a, b));
-      }
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      double2 s = C.e[i * 3 + j];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) s = cmadd(s, A.e[i * 3 + k], B.e[k * 3 + j]);
       r.e[i * 3 + j] = s;
     }
   return r;
 }
-__device__ __forceinline__ M3 msub(const M3 &A, const M3 &B) {
-  M3 r;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) r.e[k] = csub(A.e[k], B.e[k]);
-  return r;
-}
+// one step along mu, d = +-1; mu may vary at run time (no indexed arrays)
 __device__ __forceinline__ void shiftc(const Geom &g, const int x[4], int mu, int d, int o[4]) {
-  o[0] = x[0]; o[1] = x[1]; o[2] = x[2]; o[3] = x[3];
-  o[mu] = (x[mu] + d + g.L[mu]) % g.L[mu];
-}
-
-// v(y) = staple_up(y) - staple_down(y) in the (mu, nu) plane:
-//   staple_up(y)   = U_nu(y+mu) U_mu(y+nu)^dag U_nu(y)^dag
-//   staple_down(y) = U_nu(y-nu+mu)^dag U_mu(y-nu)^dag U_nu(y-nu)
-__device__ M3 staple_diff(const double2 *U, const Geom &g, const int y[4], int mu, int nu) {
-  int ypm[4], ypn[4], ymn[4], ymnpm[4];
-  shiftc(g, y, mu, 1, ypm);
-  shiftc(g, y, nu, 1, ypn);
-  shiftc(g, y, nu, -1, ymn);
-  shiftc(g, ymn, mu, 1, ymnpm);
-  M3 up = mm(mm(ld3(U, g, nu, ypm), ld3(U, g, mu, ypn), 1), ld3(U, g, nu, y), 1);
-  // (U_mu(y-nu) U_nu(y-nu+mu))^dag U_nu(y-nu)
-  M3 t = mm(ld3(U, g, mu, ymn), ld3(U, g, nu, ymnpm), 0);
-  M3 dn = mm(t, ld3(U, g, nu, ymn), 2);
-  return msub(up, dn);
-}
-
-// clover-leaf F_{mu nu}(x) = (Q - Q^dag)/8, Q = U_mu(x) v(x) + v(x-mu) U_mu(x-mu)
-// (lib/gpt/qcd/gauge/loops.py:162-174)
-__device__ M3 field_strength(const double2 *U, const Geom &g, const int x[4], int mu, int nu) {
-  int xm[4];
-  shiftc(g, x, mu, -1, xm);
-  M3 F = mm(ld3(U, g, mu, x), staple_diff(U, g, x, mu, nu), 0);
-  M3 F2 = mm(staple_diff(U, g, xm, mu, nu), ld3(U, g, mu, xm), 0);
-  M3 r;
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      double2 q = cadd(F.e[i * 3 + j], F2.e[i * 3 + j]);
-      double2 qa = cadd(F.e[j * 3 + i], F2.e[j * 3 + i]);
-      r.e[i * 3 + j] = cscale(csub(q, cconj(qa)), 0.125);
+  for (int m = 0; m < 4; ++m) {
+    int v = x[m];
+    if (m == mu) {
+      v += d;
+      v = v < 0 ? v + g.L[m] : v >= g.L[m] ? v - g.L[m] : v;
     }
-  return r;
+    o[m] = v;
+  }
 }
 
+// P with P - P^dag = 8 F_{mu nu}(x): the four plaquettes around x in the plane
+// (lib/gpt/qcd/gauge/loops.py:162-174), two of them as minus their adjoint, so
+// that they share their last link:
+//   [U_mu(x) U_nu(x+mu) U_mu(x+nu)^dag - U_mu(x-mu)^dag U_nu(x-mu) U_mu(x-mu+nu)] U_nu(x)^dag
+//   + [U_mu(x-mu)^dag U_nu(x-mu-nu)^dag U_mu(x-mu-nu) - U_mu(x) U_nu(x+mu-nu)^dag U_mu(x-nu)^dag] U_nu(x-nu)
+// Each step's loads follow the result of the one before it (after): taken ahead,
+// the 14 links are 504 registers.
+__device__ __forceinline__ const double2 *after(const double2 *G, const M3 &X) {
+  asm volatile("" : "+s"(G) : "v"(X.e[0].x), "v"(X.e[0].y), "v"(X.e[1].x), "v"(X.e[1].y), "v"(X.e[2].x), "v"(X.e[2].y),
+               "v"(X.e[3].x), "v"(X.e[3].y), "v"(X.e[4].x), "v"(X.e[4].y), "v"(X.e[5].x), "v"(X.e[5].y),
+               "v"(X.e[6].x), "v"(X.e[6].y), "v"(X.e[7].x), "v"(X.e[7].y), "v"(X.e[8].x), "v"(X.e[8].y));
+  return G;
+}
+__device__ __forceinline__ M3 plane_leaves(const double2 *G, const Geom &g, const int x[4], int mu, int nu) {
+  int xm[4], y[4], z[4];
+  shiftc(g, x, mu, -1, xm);
+  shiftc(g, x, mu, 1, y);
+  shiftc(g, x, nu, 1, z);
+  M3 X = mm(mm(ld3(G, g, mu, x), ld3(G, g, nu, y)), dag(ld3(G, g, mu, z)));
+  G = after(G, X);
+  shiftc(g, xm, nu, 1, z);
+  X = mma(X, neg(mm(dag(ld3(G, g, mu, xm)), ld3(G, g, nu, xm))), ld3(G, g, mu, z));
+  G = after(G, X);
+  M3 P = mm(X, dag(ld3(G, g, nu, x)));
+  G = after(G, P);
+  shiftc(g, xm, nu, -1, z);
+  X = mm(mm(dag(ld3(G, g, mu, xm)), dag(ld3(G, g, nu, z))), ld3(G, g, mu, z));
+  G = after(G, X);
+  shiftc(g, x, nu, -1, z);
+  shiftc(g, z, mu, 1, y);
+  X = mma(X, neg(mm(ld3(G, g, mu, x), dag(ld3(G, g, nu, y)))), dag(ld3(G, g, mu, z)));
+  G = after(G, X);
+  P = mma(P, X, ld3(G, g, nu, z));
+  return P;
+}
+
+// A workgroup takes the 64 half-sites of a block (one parity): wave pl < 6 the
+// field strength of plane pl at each of them, F_{mu nu} = (P - P^dag)/8,
+// anti-Hermitian: 9 reals in LDS.  Then wave ch < 2 assembles the chiral block
+// ch of the 64 sites, stores it and its inverse.  Bound by the links that leave
+// the L2 before their neighbours are done: 3.5 GB are fetched for 24^3 x 48, in
+// 745 us.  Fewer sites in flight keep more of them: with three or two waves
+// doing two or three planes each all waves would have work in the second half
+// too, but it takes 6.4 and 6.6 GB, 955 and 990 us.  One thread for all of a
+// site, links read in natural order (756 scattered 16-byte loads a site), took
+// 787 us.
+constexpr int kCloverThreads = 6 * kBlk;
 template <typename R>
-__global__ __launch_bounds__(128) void k_build_clover(Geom g, const double2 *U, CloverParams cp,
-                                                      typename c2<R>::t *A0, typename c2<R>::t *A1,
-                                                      typename c2<R>::t *I0, typename c2<R>::t *I1,
-                                                      int *err) {
+__global__ __launch_bounds__(kCloverThreads, 3) void k_build_clover(Geom g, const double2 *G, CloverParams cp,
+                                                                    typename c2<R>::t *A0, typename c2<R>::t *A1,
+                                                                    typename c2<R>::t *I0, typename c2<R>::t *I1,
+                                                                    int *err) {
   using C = typename c2<R>::t;
-  long i = (long)blockIdx.x * 128 + threadIdx.x;
-  if (i >= g.V) return;
-  long r = i / g.L[0];
+  __shared__ double fs[6 * 9 * kBlk];  // [plane][Im F_00, F_11, F_22, then F_10, F_20, F_21][site]
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const long nb = g.Vh / kBlk, t = xcd_tile(blockIdx.x, 2 * nb);
+  // the two parities of a block of 128 sites one after the other: they read
+  // the same links
+  const int p = (int)(t & 1);
+  const long h = (t >> 1) * kBlk + lane;
   int x[4];
-  x[0] = (int)(i - r * g.L[0]);
-  long r2 = r / g.L[1];
-  x[1] = (int)(r - r2 * g.L[1]);
-  long r3 = r2 / g.L[2];
-  x[2] = (int)(r2 - r3 * g.L[2]);
-  x[3] = (int)r3;
-  const int p = (x[0] + x[1] + x[2] + x[3]) & 1;
-  const long h = i >> 1;
+  half_coords(g, h, p, x);
   const int T = g.L[3];
   const bool edge = cp.open_bc && (x[3] == 0 || x[3] == T - 1);
   const bool next = cp.open_bc && cp.cF != 1.0 && (x[3] == 1 || x[3] == T - 2);
-
-  // B[chir][6x6] (full Hermitian, only lower + diag used)
-  double2 B[2][36];
+  if (cp.coef[w] != 0.0) {
+    const int mu = w < 3 ? 0 : w < 5 ? 1 : 2, nu = w < 3 ? w + 1 : w < 5 ? w - 1 : 3;
+    const M3 Q = plane_leaves(G, g, x, mu, nu);
+    double *f = fs + w * 9 * kBlk + lane;
+    int k = 3;
 #pragma unroll
-  for (int k = 0; k < 36; ++k) {
-    B[0][k] = make_double2(0.0, 0.0);
-    B[1][k] = make_double2(0.0, 0.0);
-  }
-  if (!edge) {
-    int pl = 0;
-    for (int mu = 0; mu < 4; ++mu)
-      for (int nu = mu + 1; nu < 4; ++nu, ++pl) {
-        if (cp.coef[pl] == 0.0) continue;
-        M3 F = field_strength(U, g, x, mu, nu);
+    for (int i = 0; i < 3; ++i) {
+      f[i * kBlk] = (Q.e[i * 4].y + Q.e[i * 4].y) * 0.125;
 #pragma unroll
-        for (int ch = 0; ch < 2; ++ch)
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-              double2 sg = make_double2(cp.sig[pl][ch][a * 2 + b][0], cp.sig[pl][ch][a * 2 + b][1]);
-              sg = cscale(sg, cp.coef[pl]);
-#pragma unroll
-              for (int c1 = 0; c1 < 3; ++c1)
-#pragma unroll
-                for (int c2_ = 0; c2_ < 3; ++c2_) {
-                  int ii = a * 3 + c1, jj = b * 3 + c2_;
-                  B[ch][ii * 6 + jj] = cadd(B[ch][ii * 6 + jj], cmul(sg, F.e[c1 * 3 + c2_]));
-                }
-            }
+      for (int j = 0; j < i; ++j, k += 2) {
+        const double2 d = cscale(csub(Q.e[i * 3 + j], cconj(Q.e[j * 3 + i])), 0.125);
+        f[k * kBlk] = d.x;
+        f[(k + 1) * kBlk] = d.y;
       }
+    }
+  }
+  __syncthreads();
+  if (w >= 2) return;
+  const int ch = w;
+  // the block: lower triangle, full Hermitian index ii = 3 a + c1
+  double2 B[36];
+#pragma unroll
+  for (int k = 0; k < 36; ++k) B[k] = make_double2(0.0, 0.0);
+  if (!edge) {
+#pragma unroll 1
+    for (int pl = 0; pl < 6; ++pl) {
+      if (cp.coef[pl] == 0.0) continue;
+      const double *f = fs + pl * 9 * kBlk + lane;
+      M3 F;
+      int k = 3;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        F.e[i * 4] = make_double2(0.0, f[i * kBlk]);
+#pragma unroll
+        for (int j = 0; j < i; ++j, k += 2) {
+          F.e[i * 3 + j] = make_double2(f[k * kBlk], f[(k + 1) * kBlk]);
+          F.e[j * 3 + i] = make_double2(-F.e[i * 3 + j].x, F.e[i * 3 + j].y);
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b <= a; ++b) {
+          double2 sg = make_double2(cp.sig[pl][ch][a * 2 + b][0], cp.sig[pl][ch][a * 2 + b][1]);
+          sg = cscale(sg, cp.coef[pl]);
+#pragma unroll
+          for (int c1 = 0; c1 < 3; ++c1)
+#pragma unroll
+            for (int c2_ = 0; c2_ < 3; ++c2_) {
+              const int ii = a * 3 + c1, jj = b * 3 + c2_;
+              if (jj <= ii) B[ii * 6 + jj] = cadd(B[ii * 6 + jj], cmul(sg, F.e[c1 * 3 + c2_]));
+            }
+        }
+    }
   }
   double dg = cp.diag;
   if (edge) dg += -0.5 * cp.csw_t;
   if (next) dg += cp.cF - 1.0;
 #pragma unroll
-  for (int ch = 0; ch < 2; ++ch)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) B[ch][k * 7].x += dg;
+  for (int k = 0; k < 6; ++k) B[k * 7].x += dg;
 
   C *A = p ? A1 : A0;
   C *Ai = p ? I1 : I0;
-#pragma unroll
-  for (int ch = 0; ch < 2; ++ch) {
-    // store A (packed), unless only the inverse is wanted
-    if (A) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        A[aidx(ch * 18 + k, h, 36)] = cmk<C>((R)B[ch][(2 * k) * 7].x, (R)B[ch][(2 * k + 1) * 7].x);
-#pragma unroll
-      for (int ii = 1; ii < 6; ++ii)
-#pragma unroll
-        for (int jj = 0; jj < ii; ++jj) {
-          double2 v = B[ch][ii * 6 + jj];
-          A[aidx(ch * 18 + tri(ii, jj), h, 36)] = cmk<C>((R)v.x, (R)v.y);
-        }
-    }
-    // LDL^H: B = L D L^H (L unit lower)
-    double d[6];
-    double2 L[36];
-    double scale = 0.0;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) scale = fmax(scale, fabs(B[ch][k * 7].x));
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-      double dj = B[ch][j * 7].x;
-#pragma unroll
-      for (int k = 0; k < j; ++k) {
-        double2 l = L[j * 6 + k];
-        dj -= (l.x * l.x + l.y * l.y) * d[k];
-      }
-      if (!(fabs(dj) > 1e-12 * scale)) {
-        *err = 1;
-        dj = 1.0;
-      }
-      d[j] = dj;
-#pragma unroll
-      for (int ii = j + 1; ii < 6; ++ii) {
-        double2 s = B[ch][ii * 6 + j];
-#pragma unroll
-        for (int k = 0; k < j; ++k) s = csub(s, cscale(cmulc(L[j * 6 + k], L[ii * 6 + k]), d[k]));
-        // s - sum L_ik conj(L_jk) d_k  (cmulc gives conj(L_jk) * L_ik)
-        L[ii * 6 + j] = cscale(s, 1.0 / dj);
-      }
-    }
-    // M = L^-1 (unit lower)
-    double2 M[36];
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-#pragma unroll
-      for (int ii = j + 1; ii < 6; ++ii) {
-        double2 s = L[ii * 6 + j];
-#pragma unroll
-        for (int k = j + 1; k < ii; ++k) s = cadd(s, cmul(L[ii * 6 + k], M[k * 6 + j]));
-        M[ii * 6 + j] = make_double2(-s.x, -s.y);
-      }
-    }
-    // (B^-1)_ij = sum_{k >= i} conj(M_ki) M_kj / d_k  for i >= j (M_kk = 1)
-#pragma unroll
-    for (int ii = 0; ii < 6; ++ii)
-#pragma unroll
-      for (int jj = 0; jj <= ii; ++jj) {
-        double2 s = make_double2(0.0, 0.0);
-#pragma unroll
-        for (int k = ii; k < 6; ++k) {
-          double2 mki = (k == ii) ? make_double2(1.0, 0.0) : M[k * 6 + ii];
-          double2 mkj = (k == jj) ? make_double2(1.0, 0.0) : M[k * 6 + jj];
-          s = cadd(s, cscale(cmulc(mki, mkj), 1.0 / d[k]));
-        }
-        if (ii == jj) {
-          B[ch][ii * 7] = s;  // B's diagonal is dead: keep the inverse's diagonal there
-        } else {
-          Ai[aidx(ch * 18 + tri(ii, jj), h, 36)] = cmk<C>((R)s.x, (R)s.y);
-        }
-      }
+  // store A (packed), unless only the inverse is wanted
+  if (A) {
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      Ai[aidx(ch * 18 + k, h, 36)] = cmk<C>((R)B[ch][(2 * k) * 7].x, (R)B[ch][(2 * k + 1) * 7].x);
+      A[aidx(ch * 18 + k, h, 36)] = cmk<C>((R)B[(2 * k) * 7].x, (R)B[(2 * k + 1) * 7].x);
+#pragma unroll
+    for (int ii = 1; ii < 6; ++ii)
+#pragma unroll
+      for (int jj = 0; jj < ii; ++jj) {
+        double2 v = B[ii * 6 + jj];
+        A[aidx(ch * 18 + tri(ii, jj), h, 36)] = cmk<C>((R)v.x, (R)v.y);
+      }
   }
+  // LDL^H: B = L D L^H (L unit lower), L in B's place
+  double d[6];
+  double scale = 0.0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) scale = fmax(scale, fabs(B[k * 7].x));
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    double dj = B[j * 7].x;
+#pragma unroll
+    for (int k = 0; k < j; ++k) {
+      double2 l = B[j * 6 + k];
+      dj -= (l.x * l.x + l.y * l.y) * d[k];
+    }
+    if (!(fabs(dj) > 1e-12 * scale)) {
+      *err = 1;
+      dj = 1.0;
+    }
+    d[j] = dj;
+#pragma unroll
+    for (int ii = j + 1; ii < 6; ++ii) {
+      double2 s = B[ii * 6 + j];
+#pragma unroll
+      for (int k = 0; k < j; ++k) s = csub(s, cscale(cmulc(B[j * 6 + k], B[ii * 6 + k]), d[k]));
+      // s - sum L_ik conj(L_jk) d_k  (cmulc gives conj(L_jk) * L_ik)
+      B[ii * 6 + j] = cscale(s, 1.0 / dj);
+    }
+  }
+  // M = L^-1 (unit lower), column by column in L's place: column j needs L's
+  // columns from j on
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+#pragma unroll
+    for (int ii = j + 1; ii < 6; ++ii) {
+      double2 s = B[ii * 6 + j];
+#pragma unroll
+      for (int k = j + 1; k < ii; ++k) s = cadd(s, cmul(B[ii * 6 + k], B[k * 6 + j]));
+      B[ii * 6 + j] = make_double2(-s.x, -s.y);
+    }
+  }
+  // (B^-1)_ij = sum_{k >= i} conj(M_ki) M_kj / d_k  for i >= j (M_kk = 1)
+  double di[6];
+#pragma unroll
+  for (int ii = 0; ii < 6; ++ii)
+#pragma unroll
+    for (int jj = 0; jj <= ii; ++jj) {
+      double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int k = ii; k < 6; ++k) {
+        double2 mki = (k == ii) ? make_double2(1.0, 0.0) : B[k * 6 + ii];
+        double2 mkj = (k == jj) ? make_double2(1.0, 0.0) : B[k * 6 + jj];
+        s = cadd(s, cscale(cmulc(mki, mkj), 1.0 / d[k]));
+      }
+      if (ii == jj) di[ii] = s.x;
+      else Ai[aidx(ch * 18 + tri(ii, jj), h, 36)] = cmk<C>((R)s.x, (R)s.y);
+    }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) Ai[aidx(ch * 18 + k, h, 36)] = cmk<C>((R)di[2 * k], (R)di[2 * k + 1]);
 }
 
 template <typename R>
-void build_clover(const Geom &g, const void *Unat, const CloverParams &cp, void *A0, void *A1, void *Ai0,
+void build_clover(const Geom &g, const void *G, const CloverParams &cp, void *A0, void *A1, void *Ai0,
                   void *Ai1, int *err_flag, hipStream_t s) {
   using C = typename c2<R>::t;
-  k_build_clover<R><<<(int)((g.V + 127) / 128), 128, 0, s>>>(g, (const double2 *)Unat, cp, (C *)A0, (C *)A1,
-                                                            (C *)Ai0, (C *)Ai1, err_flag);
+  k_build_clover<R><<<(unsigned)(2 * g.Vh / kBlk), kCloverThreads, 0, s>>>(g, (const double2 *)G, cp, (C *)A0, (C *)A1,
+                                                                          (C *)Ai0, (C *)Ai1, err_flag);
 }
 template void build_clover<double>(const Geom &, const void *, const CloverParams &, void *, void *, void *,
                                    void *, int *, hipStream_t);

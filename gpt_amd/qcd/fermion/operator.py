@@ -134,7 +134,14 @@ class interface:
     def update(self, params, U):
         if self.obj is None:
             self._setup(*self.setup_arguments)
-        _lib.check(_lib.load().wc_update(self.obj, gauge.stacked(U).data_ptr(), core.stream_ptr()))
+        # the four fields as they are, where they are contiguous on the device
+        n = 9 * self.setup_arguments[0].gsites
+        if len(U) == 4 and all(u.data.dtype == torch.complex128 and u.data.is_contiguous() and u.data.numel() == n
+                               and u.data.device == core.device()
+                               and not (u.data.is_conj() or u.data.is_neg()) for u in U):
+            _lib.check(_lib.load().wc_update_links(self.obj, *[u.data.data_ptr() for u in U], core.stream_ptr()))
+        else:
+            _lib.check(_lib.load().wc_update(self.obj, gauge.stacked(U).data_ptr(), core.stream_ptr()))
 
     def apply_unary_operator(self, opcode, dst, src):
         assert self.obj is not None

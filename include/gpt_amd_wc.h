@@ -77,6 +77,9 @@ typedef struct wc_solver_stats {
 int wc_create(const wc_params *p, const void *U, void *stream, wc_operator **out);
 /* update_fermion_operator (operators.cc:59-70, implementation.h:77-86) */
 int wc_update(wc_operator *op, const void *U, void *stream);
+/* the same from four fields [V][3][3], one per direction, as a caller holds
+ * them: no [4][V][3][3] copy of them has to be made first */
+int wc_update_links(wc_operator *op, const void *U0, const void *U1, const void *U2, const void *U3, void *stream);
 /* set_mass_fermion_operator (operators.cc:72-83, implementation.h:21-29);
  * rebuilds A and A^-1 for the new mass */
 int wc_set_mass(wc_operator *op, double mass, void *stream);

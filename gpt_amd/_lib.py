@@ -77,6 +77,8 @@ SIGNATURES = {
     "wc_trim": (_I, [_P]),
     "wc_release_cached_memory": (_I, [_P]),
     "wc_gauge_observables": (_I, [_P, _P, _P, _P, _P]),
+    "wc_site_trace": (_I, [_I, _L, _P, _P, _P, _P]),
+    "wc_slice_sum": (_I, [_L, _I, _L, _P, _P, _P, _P]),
     "wc_halo_pack": (_I, [_P, _I, _I, _I, _P, _P, _P, _P]),
     "wc_halo_unpack": (_I, [_P, _I, _I, _I, _P, _P, _P, _P]),
     "wc_bandwidth_probe": (_I, [_I, _P, _P, _L, _P]),

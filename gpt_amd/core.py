@@ -427,11 +427,24 @@ class site_scalar:
         return self.data.cpu().numpy().reshape(tuple(reversed(self.grid.fdimensions)))
 
 
+def _plain(t, dtype):
+    """whether a kernel can take the values of t as they lie in memory"""
+    return (t.dtype == dtype and t.is_contiguous() and t.device == device()
+            and not (t.is_conj() or t.is_neg() or t.requires_grad))
+
+
 def trace(x):
     """g.trace of an mspincolor (the 12 x 12 trace per site) or of a site
     product A * g.adj(B): tr(A B^dag) = sum_ij A_ij conj(B_ij), elementwise"""
     # sums in complex128 whatever the field's precision
     if isinstance(x, _site_product):
+        a, b = x.a.data, x.b.data
+        prec = {torch.complex128: double, torch.complex64: single}.get(a.dtype)
+        if prec is not None and a.shape == b.shape and a[0].numel() == 144 and _plain(a, a.dtype) and _plain(b, a.dtype):
+            out = torch.empty(a.shape[0], dtype=torch.complex128, device=a.device)
+            _lib.check(_lib.load().wc_site_trace(prec.code, a.shape[0], a.data_ptr(), b.data_ptr(), out.data_ptr(),
+                                                 stream_ptr()))
+            return site_scalar(x.a.grid, out)
         a, b = x.a.data.to(torch.complex128), x.b.data.to(torch.complex128)
         return site_scalar(x.a.grid, (a * b.conj()).reshape(a.shape[0], -1).sum(dim=1))
     if isinstance(x, mspincolor_lattice):
@@ -446,6 +459,14 @@ def slice_(x, dim):
     if not isinstance(x, site_scalar):
         raise NotImplementedError("g.slice is provided for g.trace results")
     L = x.grid.fdimensions
+    inner = int(np.prod(L[:dim])) if 0 <= dim < 4 else 0
+    # runs of less than 128 bytes (slices in x) are left to the general sum
+    if inner >= 8 and x.data.numel() == int(np.prod(L)) and _plain(x.data, torch.complex128):
+        n = L[dim]
+        work = torch.empty((17, n), dtype=torch.complex128, device=x.data.device)
+        _lib.check(_lib.load().wc_slice_sum(x.data.numel() // (n * inner), n, inner, x.data.data_ptr(),
+                                            work[1].data_ptr(), work.data_ptr(), stream_ptr()))
+        return [complex(c) for c in work[0].cpu().numpy()]
     v = x.data.reshape(L[3], L[2], L[1], L[0])
     other = tuple(d for d in range(4) if d != 3 - dim)
     return [complex(c) for c in v.sum(dim=other).cpu().numpy()]

@@ -1480,6 +1480,23 @@ int wc_gauge_observables(const int fdims[4], const void *U, double *plaquette, d
   return WC_OK;
 }
 
+int wc_site_trace(int prec, long n, const void *a, const void *b, void *out, void *stream) {
+  WC_PREC_CHECK(prec);
+  if (n < 0 || (n > 0 && (!a || !b || !out))) WC_FAIL(WC_ERR_ARG, "wc_site_trace: bad arguments");
+  hipStream_t s = (hipStream_t)stream;
+  if (prec == WC_DOUBLE) wck::site_trace<double>(n, a, b, out, s);
+  else wck::site_trace<float>(n, a, b, out, s);
+  WC_LAUNCHED();
+  return WC_OK;
+}
+
+int wc_slice_sum(long outer, int n, long inner, const void *f, void *work, void *out, void *stream) {
+  if (outer < 1 || n < 1 || inner < 1 || !f || !work || !out) WC_FAIL(WC_ERR_ARG, "wc_slice_sum: bad arguments");
+  wck::slice_sum(outer, n, inner, f, work, out, (hipStream_t)stream);
+  WC_LAUNCHED();
+  return WC_OK;
+}
+
 int wc_field_export(const int fdims[4], int prec, const void *eo, void *natural, void *stream) {
   WC_PREC_CHECK(prec);
   Geom g;

@@ -153,6 +153,13 @@ void reduce_final(const double *partials, int n, double *out, hipStream_t s);
 // plaquettes and of Re tr of the 4 links
 void gauge_obs_partials(const Geom &g, const void *U, double *pplaq, double *ptrace, hipStream_t s);
 
+// the site-wise trace of A B^dag of two propagators (144 entries a site) and
+// the sums of a complex FP64 field (outer, n, inner) over outer and inner; part
+// holds kSliceParts * n complex values
+constexpr int kSliceParts = 16;
+template <typename R> void site_trace(long n, const void *a, const void *b, void *out, hipStream_t s);
+void slice_sum(long outer, int n, long inner, const void *f, void *part, void *out, hipStream_t s);
+
 // precision conversion of n complex entries
 void convert_d2f(long n, const void *src, void *dst, hipStream_t s);
 void convert_f2d(long n, const void *src, void *dst, hipStream_t s);

@@ -401,6 +401,14 @@ int wc_halo_interior(wc_operator *op, int parity_out, int dag, int nrhs, void *d
  * NERSC configuration reader and writer (gpt_amd/io.py). */
 int wc_gauge_observables(const int fdims[4], const void *U, double *plaquette, double *link_trace, void *stream);
 
+/* contractions of a propagator, natural [sites][144] (gpt's mspincolor):
+ * out[x] = sum_k a[x][k] conj(b[x][k]), g.trace(a * g.adj(b)), complex FP64 from
+ * either precision; and the sums of a complex FP64 field of shape
+ * (outer, n, inner) over outer and inner, g.slice, with room for 16 n complex
+ * FP64 values in work */
+int wc_site_trace(int prec, long sites, const void *a, const void *b, void *out, void *stream);
+int wc_slice_sum(long outer, int n, long inner, const void *field, void *work, void *out, void *stream);
+
 /* HBM bandwidth probe (no counterpart in the reference; a measurement
  * utility): kind 0 copies `bytes` from src to dst, kind 1 only reads src (and
  * writes a 32 KB XOR fold to dst, so bytes >= 32768); both stream 16 bytes

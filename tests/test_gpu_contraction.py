@@ -1,0 +1,82 @@
+"""g.trace(a * g.adj(b)) and g.slice against numpy in extended precision: both
+field precisions, a field with itself and with another, ragged lattices (sites
+not a multiple of a wave's), every direction, infinities, and the forms that
+the general path takes (views, mixed precisions)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():  # pragma: no cover
+    pytest.skip("no GPU", allow_module_level=True)
+
+import gpt_amd as g  # noqa: E402
+
+L = np.clongdouble
+
+
+def prop(grid, seed):
+    p = g.mspincolor(grid)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    p.data.copy_(torch.randn(p.data.shape, generator=gen, device="cuda", dtype=p.data.dtype))
+    return p
+
+
+def reference(a, b):
+    return (a.data.cpu().numpy().astype(L) * b.data.cpu().numpy().astype(L).conj()).reshape(a.data.shape[0], -1).sum(1)
+
+
+def check(got, want, scale, terms):
+    """FP64 sums of `terms` products of sum of magnitudes `scale`, in any order"""
+    assert np.all(np.abs(got - want) <= (terms + 4) * 2.3e-16 * scale)
+
+
+@pytest.mark.parametrize("prec", [g.double, g.single], ids=["double", "single"])
+@pytest.mark.parametrize("fd", [[4, 4, 4, 4], [2, 4, 16, 4], [6, 10, 32, 2], [12, 8, 8, 6], [16, 8, 2, 26]], ids=str)
+def test_trace_and_slices(fd, prec):
+    grid = g.grid(fd, prec)
+    a, b = prop(grid, 1), prop(grid, 2)
+    for x, y in ((a, a), (a, b), (b, a)):
+        tr = g.trace(x * g.adj(y))
+        assert tr.data.dtype == torch.complex128
+        want = reference(x, y)
+        mag = np.abs(x.data.cpu().numpy().astype(L) * y.data.cpu().numpy().astype(L)).reshape(len(want), -1).sum(1)
+        check(tr.data.cpu().numpy(), want, mag, 144)
+        if x is y:
+            assert float(tr.data.imag.abs().max()) == 0
+        f = tr.data.cpu().numpy().astype(L).reshape(fd[::-1])
+        for dim in range(4):
+            other = tuple(d for d in range(4) if d != 3 - dim)
+            check(np.array(g.slice(tr, dim)), f.sum(other), np.abs(f).sum(other), f.size // fd[dim])
+
+
+def test_forms_of_the_general_path_agree():
+    grid, gs = g.grid([4, 6, 8, 4], g.double), g.grid([4, 6, 8, 4], g.single)
+    a, b, c = prop(grid, 1), prop(grid, 2), prop(gs, 3)
+    want = g.trace(a * g.adj(b)).data
+    mag = 144 * 40.0
+    v = g.mspincolor(grid)
+    v.data = torch.stack([b.data, b.data], -1)[..., 1]  # strided
+    assert float((g.trace(a * g.adj(v)).data - want).abs().max()) < 1e-16 * mag * 144
+    v.data = b.data.conj().clone().conj()  # a lazy conjugate
+    assert v.data.is_conj()
+    assert float((g.trace(a * g.adj(v)).data - want).abs().max()) < 1e-16 * mag * 144
+    got = g.trace(a * g.adj(c)).data.cpu().numpy()  # mixed precisions
+    ref = reference(a, c)
+    assert np.all(np.abs(got - ref) < 1e-16 * mag * 144)
+    off = torch.empty(c.data.numel() + 1, dtype=torch.complex64, device="cuda")[1:].view(c.data.shape)
+    off.copy_(c.data)  # 8 bytes off
+    u = g.mspincolor(gs)
+    u.data = off
+    assert torch.equal(g.trace(u * g.adj(u)).data, g.trace(c * g.adj(c)).data)
+
+
+def test_infinities_stay_in_their_slice():
+    grid = g.grid([4, 4, 8, 6], g.double)
+    a = prop(grid, 1)
+    fin = g.slice(g.trace(a * g.adj(a)), 3)
+    a.data[3 * 128 + 5, 1, 2, 0, 1] = float("inf")
+    got = g.slice(g.trace(a * g.adj(a)), 3)
+    assert got[3].real == float("inf") or np.isnan(got[3].real)
+    assert [x for t, x in enumerate(got) if t != 3] == [x for t, x in enumerate(fin) if t != 3]

@@ -59,6 +59,8 @@ SIGNATURES = {
     "wc_norm2": (_I, [_I, _L, _P, ctypes.POINTER(_D), _P]),
     "wc_inner_product": (_I, [_I, _L, _P, _P, ctypes.POINTER(_D), _P]),
     "wc_axpy_norm2": (_I, [_I, _L, _D, _D, _P, _P, _P, ctypes.POINTER(_D), _P]),
+    "wc_pack_rhs": (_I, [_I, _L, _I, _P, _P, _P]),
+    "wc_unpack_rhs": (_I, [_I, _L, _I, _P, _P, _P]),
     "wc_convert": (_I, [_I, _P, _I, _P, _L, _P]),
     "wc_field_import": (_I, [ctypes.POINTER(_I), _I, _P, _P, _P]),
     "wc_field_export": (_I, [ctypes.POINTER(_I), _I, _P, _P, _P]),

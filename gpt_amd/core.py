@@ -427,7 +427,7 @@ class site_scalar:
         return self.data.cpu().numpy().reshape(tuple(reversed(self.grid.fdimensions)))
 
 
-def _plain(t, dtype):
+def plain(t, dtype):
     """whether a kernel can take the values of t as they lie in memory"""
     return (t.dtype == dtype and t.is_contiguous() and t.device == device()
             and not (t.is_conj() or t.is_neg() or t.requires_grad))
@@ -440,7 +440,7 @@ def trace(x):
     if isinstance(x, _site_product):
         a, b = x.a.data, x.b.data
         prec = {torch.complex128: double, torch.complex64: single}.get(a.dtype)
-        if prec is not None and a.shape == b.shape and a[0].numel() == 144 and _plain(a, a.dtype) and _plain(b, a.dtype):
+        if prec is not None and a.shape == b.shape and a[0].numel() == 144 and plain(a, a.dtype) and plain(b, a.dtype):
             out = torch.empty(a.shape[0], dtype=torch.complex128, device=a.device)
             _lib.check(_lib.load().wc_site_trace(prec.code, a.shape[0], a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                                  stream_ptr()))
@@ -461,7 +461,7 @@ def slice_(x, dim):
     L = x.grid.fdimensions
     inner = int(np.prod(L[:dim])) if 0 <= dim < 4 else 0
     # runs of less than 128 bytes (slices in x) are left to the general sum
-    if inner >= 8 and x.data.numel() == int(np.prod(L)) and _plain(x.data, torch.complex128):
+    if inner >= 8 and x.data.numel() == int(np.prod(L)) and plain(x.data, torch.complex128):
         n = L[dim]
         work = torch.empty((17, n), dtype=torch.complex128, device=x.data.device)
         _lib.check(_lib.load().wc_slice_sum(x.data.numel() // (n * inner), n, inner, x.data.data_ptr(),

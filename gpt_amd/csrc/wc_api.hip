@@ -1497,6 +1497,27 @@ int wc_slice_sum(long outer, int n, long inner, const void *f, void *work, void 
   return WC_OK;
 }
 
+static int pack_call(int prec, long n, int nrhs, void *const *fields, void *packed, int unpack, void *stream) {
+  WC_PREC_CHECK(prec);
+  const char *name = unpack ? "wc_unpack_rhs" : "wc_pack_rhs";
+  if (n < 0 || nrhs < 1 || nrhs > 64 || !fields || (n > 0 && !packed)) WC_FAIL(WC_ERR_ARG, "%s: bad arguments", name);
+  for (int r = 0; r < nrhs; ++r)
+    if (n > 0 && !fields[r]) WC_FAIL(WC_ERR_ARG, "%s: field %d is null", name, r);
+  hipStream_t s = (hipStream_t)stream;
+  if (prec == WC_DOUBLE) wck::pack_rhs<double>(n, nrhs, fields, packed, unpack, s);
+  else wck::pack_rhs<float>(n, nrhs, fields, packed, unpack, s);
+  WC_LAUNCHED();
+  return WC_OK;
+}
+
+int wc_pack_rhs(int prec, long n, int nrhs, const void *const *fields, void *packed, void *stream) {
+  return pack_call(prec, n, nrhs, (void *const *)fields, packed, 0, stream);
+}
+
+int wc_unpack_rhs(int prec, long n, int nrhs, const void *packed, void *const *fields, void *stream) {
+  return pack_call(prec, n, nrhs, fields, (void *)packed, 1, stream);
+}
+
 int wc_field_export(const int fdims[4], int prec, const void *eo, void *natural, void *stream) {
   WC_PREC_CHECK(prec);
   Geom g;

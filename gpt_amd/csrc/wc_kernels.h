@@ -168,6 +168,11 @@ void convert_f2d(long n, const void *src, void *dst, hipStream_t s);
 template <typename R> void import_field(const Geom &g, const void *nat, void *eo, hipStream_t s);
 template <typename R> void export_field(const Geom &g, const void *eo, void *nat, hipStream_t s);
 
+// fields of n complex entries to or from one field of N right-hand sides
+// (N <= 64), kPackRhs of them to a workgroup
+constexpr int kPackRhs = 32;
+template <typename R> void pack_rhs(long n, int N, void *const *fields, void *packed, int unpack, hipStream_t s);
+
 // operator set-up from natural FP64 links [V][9], one device pointer a
 // direction: the kept gauge field G (FP64, 36 V complex, blocked by parity) and
 // the hop's links

@@ -513,12 +513,35 @@ def wilson_clover(U, params=None, **kwargs):
     return fine_operator("wilson_clover", U, p)
 
 
+def _pointers(fields, packed, written):
+    """the fields' addresses, if one kernel can move them to or from the packed
+    field: as they lie in memory, of its precision and geometry, and, where they
+    are written, apart from each other and from it"""
+    t = packed.data
+    shape = t.shape[:-2] + (1, 2)
+    if len(fields) < 2 or not core.plain(t, t.dtype):
+        return None
+    if not all(f.data.shape == shape and core.plain(f.data, t.dtype) for f in fields):
+        return None
+    ptrs = [f.data.data_ptr() for f in fields]
+    if written:
+        size = fields[0].data.numel() * t.element_size()
+        ends = sorted([(p, p + size) for p in ptrs] + [(t.data_ptr(), t.data_ptr() + size * len(ptrs))])
+        if any(b[0] < a[1] for a, b in zip(ends, ends[1:])):
+            return None
+    return (ctypes.c_void_p * len(ptrs))(*ptrs)
+
+
 def pack(fields, g=None):
     """list of single-RHS fields -> one multi-RHS field (RHS innermost)"""
     n = len(fields)
     g = (g or fields[0].grid).inserted_dimension(n)
     out = lattice(g)
     out._cb = fields[0].checkerboard()
+    ptrs = _pointers(fields, out, False)
+    if ptrs is not None and all(f.grid.nrhs == 1 and f.grid.Vh == g.Vh and f.grid.cb is g.cb for f in fields):
+        _lib.check(_lib.load().wc_pack_rhs(g.precision.code, out.nentries // n, n, ptrs, out.ptr(), core.stream_ptr()))
+        return out
     for r, f in enumerate(fields):
         out.set_rhs(r, f)
     return out
@@ -527,9 +550,16 @@ def pack(fields, g=None):
 def unpack(field, dst=None):
     n = field.grid.nrhs
     if dst is None:
-        return [field.rhs(r) for r in range(n)]
+        dst = [lattice(field.grid.single_rhs()) for _ in range(n)]
+        for x in dst:
+            x._cb = field.checkerboard()
+    ptrs = _pointers(dst[:n], field, True) if len(dst) >= n else None
+    if ptrs is not None:
+        _lib.check(_lib.load().wc_unpack_rhs(field.grid.precision.code, field.nentries // n, n, field.ptr(), ptrs,
+                                             core.stream_ptr()))
     for r in range(n):
-        dst[r].data.copy_(field.data[..., r:r + 1, :])
+        if ptrs is None:
+            dst[r].data.copy_(field.data[..., r:r + 1, :])
         if dst[r].grid.cb is not full:
             dst[r].checkerboard(field.checkerboard())
     return dst

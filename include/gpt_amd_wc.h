@@ -117,6 +117,12 @@ int wc_axpy_norm2(int prec, long n, double a_re, double a_im, const void *x, con
 /* g.convert between FP64 and FP32 storage (transform.cc:128-141) */
 int wc_convert(int dst_prec, void *dst, int src_prec, const void *src, long n, void *stream);
 
+/* nrhs (<= 64) fields of n complex entries each, given by their device
+ * pointers, to one field of nrhs right-hand sides (rhs innermost) and back
+ * (matrix_operator.py:200-239); the fields must not overlap */
+int wc_pack_rhs(int prec, long n, int nrhs, const void *const *fields, void *packed, void *stream);
+int wc_unpack_rhs(int prec, long n, int nrhs, const void *packed, void *const *fields, void *stream);
+
 /* natural [V][4][3] <-> even-odd full field (layout plumbing for I/O) */
 int wc_field_import(const int fdims[4], int prec, const void *natural, void *eo, void *stream);
 int wc_field_export(const int fdims[4], int prec, const void *eo, void *natural, void *stream);

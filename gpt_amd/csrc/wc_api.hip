@@ -972,6 +972,7 @@ static int pick_s16(wc_operator *op, int N, hipStream_t s) {
   };
   const wck::HopShape base = shape_for(op, N);
   add(base, 0);
+  add(default_shape16(op, N), 0);
   for (int rb = 1; rb <= 2 && rb <= N; ++rb)
     for (int tpb : {2, 4, 8})
       for (int oc : {0, 4, 8}) {

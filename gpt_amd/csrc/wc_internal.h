@@ -290,26 +290,54 @@ inline bool stage_fits(const wc_operator *op, int nrhs, const wck::HopShape &sh)
   return bytes <= (size_t)wck::kMaxStageBytes;
 }
 
-// Shape used until the tuner (or the caller) picks one: at most 4
-// workgroups per CU; with several right-hand sides, rb per thread with the
-// least padding (ties: the larger rb), 256 threads per workgroup and the
-// links staged in LDS where the staging area fits.
+// the most waves a workgroup (a power of 2, at most `most`) with 192 workgroups of them
+inline int widest(long waves, int most) {
+  int t = 1;
+  while (2 * t <= most && waves >= 192 * 2 * t) t *= 2;
+  return t;
+}
+
+// Shape used until the tuner (or the caller) picks one.  Two things decide:
+// - whether what a hop touches stays in the 256 MB of the Infinity Cache from
+//   one hop to the next.  If so, large workgroups that still give nearly every
+//   CU one (192) are fastest; if not, the neighbours in the 4 MB L2 decide, and
+//   small ones keep them closer together.
+// - whether the items of a site share its links.  One or two items read them
+//   faster themselves than through LDS; more stage them.
+// FP32, one right-hand side: 20 x 12 x 24 x 36 (125 MB) 19.3 us with 8 waves a
+// workgroup, 22.3 with 2; 32^3 x 64 (800 MB) 154 and 145.  One wave and at most 4
+// workgroups per CU, the shape of all of them before, took 29.1 and 190.  FP64:
+// 16^3 x 32 25.0 -> 19.4 us, 32^3 x 64 266 -> 262 us.
 inline wck::HopShape default_shape(const wc_operator *op, int nrhs) {
+  const bool f64 = op->prec == WC_DOUBLE;
+  const long blocks = op->g.Vh / kBlk;
+  const bool cached = op->g.Vh * (8 * op->nl + 24 * nrhs) * (long)op->csz <= (256L << 20);
   wck::HopShape sh;
-  sh.occ = 4;
-  if (nrhs <= 1) return sh;
-  sh.tpb = 4;
-  const int mrb = max_rb_prec(op->prec);
-  int best = 1, waste_best = 1 << 30;
-  for (int rb = mrb; rb >= 1; --rb) {
-    const int waste = ((nrhs + rb - 1) / rb) * rb - nrhs;
-    if (waste < waste_best) {
-      waste_best = waste;
-      best = rb;
-    }
+  if (nrhs <= 1) {
+    // spinors staged in LDS, where a workgroup has more than one wave or the L2
+    // would have to hold them
+    sh.tpb = cached ? widest(blocks, f64 ? 4 : 8) : f64 ? 1 : 2;
+    sh.ls = sh.tpb > 1 || !cached ? 2 : 0;
+    // FP64 slices near the L2's size and whole links: 262 us against 270 for
+    // 32^3 x 64; with 12-real links or smaller slices the limit costs 5 %
+    sh.occ = f64 && op->nl == 9 && !cached && blocks > 128L * op->g.L[3] ? 4 : 0;
+  } else if (f64 && (nrhs == 2 || (nrhs == 4 && cached))) {
+    // 16^3 x 32: two right-hand sides 35.5 -> 31.4 us; 12^3 x 24: four 28 -> 23
+    sh.tpb = nrhs == 2 && cached ? widest(2 * blocks, 8) : 2;
+    sh.occ = 4;
+  } else if (!f64 && nrhs <= 4) {
+    // two right-hand sides a thread, also of an odd number (the last thread of a
+    // site then repeats one): 32^3 x 64 with two 252 -> 195 us, three 373 -> 291
+    sh.rb = 2;
+    sh.tpb = cached ? widest(nrhs > 2 ? 2 * blocks : blocks, 4) : nrhs > 2 ? 2 : 1;
+  } else {
+    // right-hand sides a thread with the least padding, links staged where the
+    // area fits
+    sh.tpb = 4;
+    sh.occ = 4;
+    sh.rb = max_rb_prec(op->prec) > 1 && nrhs % 2 == 0 ? 2 : 1;
+    sh.ls = 1;
   }
-  sh.rb = best;
-  sh.ls = 1;
   if (!stage_fits(op, nrhs, sh)) sh.ls = 0;
   return sh;
 }
@@ -352,10 +380,29 @@ inline wck::HopShape shape_for(const wc_operator *op, int nrhs) {
   return default_shape(op, nrhs);
 }
 
+// the shape of the hops with 16-bit spinors until one was timed: these are
+// bound by their arithmetic, where one right-hand side a thread and as many
+// waves as fit are fastest, links staged from 7 right-hand sides on; two and four
+// fill a thread's pairs without a rest.  Normal operator on 24^3 x 48 with
+// 12-real links: 3, 4, 5, 8 and 11 right-hand sides 469, 518, 757, 1010 and 1196
+// us in the FP32 hop's shapes, 430, 491, 645, 785 and 1087 in these.
+inline wck::HopShape default_shape16(const wc_operator *op, int nrhs) {
+  wck::HopShape sh;
+  if (nrhs <= 2) return default_shape(op, nrhs);
+  if (nrhs == 4) {
+    sh.rb = 2;
+    return sh;
+  }
+  sh.tpb = widest(op->g.Vh / kBlk * nrhs, 4);
+  sh.ls = nrhs >= 7 ? 1 : 0;
+  if (!stage_fits(op, nrhs, sh)) sh.ls = 0;
+  return sh;
+}
+
 // launch shape of the hops with 16-bit spinors (FP32 operator): the caller's
 // shape if one was set, else the one timed fastest for those hops (pick_s16,
 // process-wide per lattice, link format and class of right-hand-side
-// counts), else the FP32 hop's
+// counts), else the default
 extern std::map<ShapeKey, wck::HopShape> g_shape16_cache;
 inline wck::HopShape shape16_for(const wc_operator *op, int nrhs) {
   if (nrhs >= 1 && nrhs <= 64 && op->shape_user[nrhs]) return op->shape[nrhs];
@@ -369,7 +416,7 @@ inline wck::HopShape shape16_for(const wc_operator *op, int nrhs) {
       return sh;
     }
   }
-  return shape_for(op, nrhs);
+  return default_shape16(op, nrhs);
 }
 
 // the hop form timed faster for the operator's lattice, link format and

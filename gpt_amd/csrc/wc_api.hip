@@ -1331,14 +1331,24 @@ int wc_solve_eo2_ne(wc_operator *op, int parity, void *dst, const void *src, dou
 // ------------------------------------------------------------------ BLAS
 extern "C" {
 
-static thread_local double *g_red = nullptr;      // device partials + result
-static thread_local double *g_red_host = nullptr;  // pinned host copy
+static thread_local double *g_red = nullptr;       // device partials of up to two sums
+static thread_local double *g_red_host = nullptr;  // the sums: pinned, written by the kernel
 
 static int red_buffers() {
   if (!g_red) {
-    WC_HIP(wc_dev_malloc((void **)&g_red, sizeof(double) * (2 * wck::kRedBlocks + 4)));
-    WC_HIP(hipHostMalloc((void **)&g_red_host, sizeof(double) * 4, hipHostMallocDefault));
+    WC_HIP(wc_dev_malloc((void **)&g_red, sizeof(double) * 2 * wck::kRedBlocks));
+    WC_HIP(hipHostMalloc((void **)&g_red_host, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocPortable));
   }
+  return WC_OK;
+}
+// the sums of the kRedBlocks partials at g_red (and at g_red + kRedBlocks) to
+// g_red_host, complete on return
+static int red_sums(int sums, hipStream_t s) {
+  void *out = nullptr;
+  WC_HIP(hipHostGetDevicePointer(&out, g_red_host, 0));
+  wck::reduce_final(g_red, wck::kRedBlocks, sums, (double *)out, s);
+  WC_LAUNCHED();
+  WC_HIP(hipStreamSynchronize(s));
   return WC_OK;
 }
 
@@ -1371,14 +1381,10 @@ int wc_inner_product(int prec, long n, const void *a, const void *b, double *res
   int rc = red_buffers();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  double *pre = g_red, *pim = g_red + wck::kRedBlocks, *res = g_red + 2 * wck::kRedBlocks;
+  double *pre = g_red, *pim = g_red + wck::kRedBlocks;
   if (prec == WC_DOUBLE) wck::dot_partials<double>(n, a, b, pre, pim, s);
   else wck::dot_partials<float>(n, a, b, pre, pim, s);
-  wck::reduce_final(pre, wck::kRedBlocks, res, s);
-  wck::reduce_final(pim, wck::kRedBlocks, res + 1, s);
-  WC_LAUNCHED();
-  WC_HIP(hipMemcpyAsync(g_red_host, res, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-  WC_HIP(hipStreamSynchronize(s));
+  if ((rc = red_sums(2, s))) return rc;
   result[0] = g_red_host[0];
   result[1] = g_red_host[1];
   return WC_OK;
@@ -1390,13 +1396,10 @@ int wc_norm2(int prec, long n, const void *x, double *result, void *stream) {
   int rc = red_buffers();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  double *pre = g_red, *res = g_red + 2 * wck::kRedBlocks;
+  double *pre = g_red;
   if (prec == WC_DOUBLE) wck::norm2_partials<double>(n, x, pre, s);
   else wck::norm2_partials<float>(n, x, pre, s);
-  wck::reduce_final(pre, wck::kRedBlocks, res, s);
-  WC_LAUNCHED();
-  WC_HIP(hipMemcpyAsync(g_red_host, res, sizeof(double), hipMemcpyDeviceToHost, s));
-  WC_HIP(hipStreamSynchronize(s));
+  if ((rc = red_sums(1, s))) return rc;
   *result = g_red_host[0];
   return WC_OK;
 }
@@ -1408,13 +1411,10 @@ int wc_axpy_norm2(int prec, long n, double a_re, double a_im, const void *x, con
   int rc = red_buffers();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  double *pre = g_red, *res = g_red + 2 * wck::kRedBlocks;
+  double *pre = g_red;
   if (prec == WC_DOUBLE) wck::axpy_norm2_partials<double>(n, a_re, a_im, x, y, z, pre, s);
   else wck::axpy_norm2_partials<float>(n, a_re, a_im, x, y, z, pre, s);
-  wck::reduce_final(pre, wck::kRedBlocks, res, s);
-  WC_LAUNCHED();
-  WC_HIP(hipMemcpyAsync(g_red_host, res, sizeof(double), hipMemcpyDeviceToHost, s));
-  WC_HIP(hipStreamSynchronize(s));
+  if ((rc = red_sums(1, s))) return rc;
   *result = g_red_host[0];
   return WC_OK;
 }
@@ -1468,13 +1468,9 @@ int wc_gauge_observables(const int fdims[4], const void *U, double *plaquette, d
   if (!U || !plaquette || !link_trace) WC_FAIL(WC_ERR_ARG, "wc_gauge_observables: null argument");
   if ((rc = red_buffers())) return rc;
   hipStream_t s = (hipStream_t)stream;
-  double *pp = g_red, *pt = g_red + wck::kRedBlocks, *res = g_red + 2 * wck::kRedBlocks;
+  double *pp = g_red, *pt = g_red + wck::kRedBlocks;
   wck::gauge_obs_partials(g, U, pp, pt, s);
-  wck::reduce_final(pp, wck::kRedBlocks, res, s);
-  wck::reduce_final(pt, wck::kRedBlocks, res + 1, s);
-  WC_LAUNCHED();
-  WC_HIP(hipMemcpyAsync(g_red_host, res, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-  WC_HIP(hipStreamSynchronize(s));
+  if ((rc = red_sums(2, s))) return rc;
   // gpt's normalisation: averages of Re tr / 3 over the 6 planes and the 4 directions
   *plaquette = g_red_host[0] / (6.0 * 3.0 * (double)g.V);
   *link_trace = g_red_host[1] / (4.0 * 3.0 * (double)g.V);

@@ -146,7 +146,7 @@ template <typename R>
 void axpy_norm2_partials(long n, double ar, double ai, const void *x, const void *y, void *z,
                          double *pre, hipStream_t s);
 // out[0] = sum of partials (fixed order, one block)
-void reduce_final(const double *partials, int n, double *out, hipStream_t s);
+void reduce_final(const double *partials, int n, int sums, double *out, hipStream_t s);
 
 // gauge observables of natural FP64 links U[4][V][3][3] (periodic): per block
 // of a fixed grid (kRedBlocks), the sum over sites of Re tr of the 6

@@ -170,15 +170,17 @@ template void axpy_norm2_partials<double>(long, double, double, const void *, co
 template void axpy_norm2_partials<float>(long, double, double, const void *, const void *, void *, double *,
                                          hipStream_t);
 
+// out[b] = sum of p[b n .. b n + n), a block per sum; out may be pinned host
+// memory, which saves the copy of the sums (9 us) after the kernel (5 us)
 __global__ __launch_bounds__(1024) void k_reduce_final(const double *p, int n, double *out) {
   __shared__ double red[1024 / 64 + 1];
   double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) s += p[i];
+  for (int i = threadIdx.x; i < n; i += 1024) s += p[(long)blockIdx.x * n + i];
   s = block_sum<1024>(s, red);
-  if (threadIdx.x == 0) out[0] = s;
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
-void reduce_final(const double *partials, int n, double *out, hipStream_t s) {
-  k_reduce_final<<<1, 1024, 0, s>>>(partials, n, out);
+void reduce_final(const double *partials, int n, int sums, double *out, hipStream_t s) {
+  k_reduce_final<<<sums, 1024, 0, s>>>(partials, n, out);
 }
 
 // ------------------------------------------------------- gauge observables

@@ -88,7 +88,14 @@ def device():
     return _device
 
 
+# torch's current stream as the bare handle (0.1 us): current_stream() makes a
+# Stream object of it first (2.7 us, of the 9.5 of a hop on an 8^4 lattice)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr():
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
     return ctypes_void(torch.cuda.current_stream().cuda_stream)
 
 

@@ -147,11 +147,15 @@ __device__ __forceinline__ void compute_dir(const HopLaunch &a, const int c[4], 
   }
 }
 
-// The 8 directions run as a real loop (not unrolled): the loads of one
-// direction cannot be hoisted into another, so the live registers stay at one
-// direction's operands plus the accumulators; the other waves on the SIMD
-// keep HBM busy meanwhile.  The projection variant is picked by a
-// wave-uniform switch.  Neighbour offsets come from uniform strides of the
+// The 8 directions are unrolled, each fenced from the next: no load of one is
+// hoisted into another, so the live registers stay at one direction's operands
+// plus the accumulators; the other waves on the SIMD keep HBM busy meanwhile.
+// As a loop with a switch over the projections, every direction copied 12 of the
+// sums and chose its neighbour at run time, a quarter of the instructions of the
+// 16-bit hops, which the VALUs bound (1540 a wave at 12 right-hand sides, 90 %
+// busy), and took more registers (FP16 AXPY hop 90, now 69).  FP16 Mpc^dag Mpc at
+// 24^3 x 48: 1193 -> 1155 us; FP64 Meooe at 32^3 x 64: 276 -> 270 us.
+// Neighbour offsets come from uniform strides of the
 // half-site index h = ((t*Lz + z)*Ly + y)*Lxh + x/2.  The item's right-hand
 // sides are r0 .. r0 + RB - 1, adjacent in memory: one access of RB values
 // per component.  With one access per value, RB = 2 made 20-25 cache accesses
@@ -160,7 +164,7 @@ __device__ __forceinline__ void compute_dir(const HopLaunch &a, const int c[4], 
 // 1066 us, FP16 Mpc^dag Mpc at 24^3 x 48: 1612 -> 1230 us.
 //
 // LS: the links are staged in LDS, prepared (prepare_link), entry e of
-// direction dir of the site at lw[(dir * 9 + e) * ns].
+// direction dir of the site at lw[dir * 9 + e].
 //
 // XS: xst (non-null) holds the input spinors of the half-sites xs0 ..
 // xs0 + xsn - 1, component k of site xs0 + i at xst[k * xsl + i]; a
@@ -169,7 +173,7 @@ template <typename R, int NL, int DAG, int RB, typename SI, bool LS, bool XS>
 __device__ __forceinline__ void hop_site(const HopLaunch &a, long h, const int r0, const int cx,
                                          const int cy, const int cz, const int ct,
                                          typename c2<R>::t acc[RB][12], const typename c2<R>::t *lw,
-                                         int ns, const typename c2<R>::t *xst, long xs0, int xsn, int xsl) {
+                                         const typename c2<R>::t *xst, long xs0, int xsn, int xsl) {
   // coordinates as scalars: a select among array elements would become a
   // dynamically indexed (scratch) array
   const int c[4] = {cx, cy, cz, ct};
@@ -194,10 +198,9 @@ __device__ __forceinline__ void hop_site(const HopLaunch &a, long h, const int r
   const uint32_t kstride = (uint32_t)kBlk * N * (uint32_t)sizeof(SI);
   const uint32_t xh = (uint32_t)cx >> 1;
   const uint32_t st1 = (uint32_t)g.Lxh, st2 = st1 * (uint32_t)g.L[1], st3 = st2 * (uint32_t)g.L[2];
-#pragma unroll 1
-  for (int dir = 0; dir < 8; ++dir) {
-    const int mu = dir >> 1, fb = dir & 1;
-    if (mu == 3 && a.skip_t_faces && (fb == 0 ? ct == g.L[3] - 1 : ct == 0)) continue;
+  auto one = [&](auto D) {
+    constexpr int dir = decltype(D)::value, mu = dir >> 1, fb = dir & 1;
+    if (mu == 3 && a.skip_t_faces && (fb == 0 ? ct == g.L[3] - 1 : ct == 0)) return;
     uint32_t nb;
     if (mu == 0) {
       const int xn = fb == 0 ? (cx == g.L[0] - 1 ? 0 : cx + 1) : (cx == 0 ? g.L[0] - 1 : cx - 1);
@@ -215,7 +218,7 @@ __device__ __forceinline__ void hop_site(const HopLaunch &a, long h, const int r
     C u[9];
     if constexpr (LS) {
 #pragma unroll
-      for (int e = 0; e < 9; ++e) u[e] = lw[(dir * 9 + e) * ns];
+      for (int e = 0; e < 9; ++e) u[e] = lw[dir * 9 + e];
     } else {
       const uint32_t dsoff = (uint32_t)(dir * NL) * (uint32_t)(kBlk * sizeof(C));
 #pragma unroll
@@ -257,17 +260,22 @@ __device__ __forceinline__ void hop_site(const HopLaunch &a, long h, const int r
         }
       }
     }
-    switch (dir) {
-      case 0: compute_dir<R, NL, DAG, 0, 0, RB, LS>(a, c, u, psi, acc); break;
-      case 1: compute_dir<R, NL, DAG, 0, 1, RB, LS>(a, c, u, psi, acc); break;
-      case 2: compute_dir<R, NL, DAG, 1, 0, RB, LS>(a, c, u, psi, acc); break;
-      case 3: compute_dir<R, NL, DAG, 1, 1, RB, LS>(a, c, u, psi, acc); break;
-      case 4: compute_dir<R, NL, DAG, 2, 0, RB, LS>(a, c, u, psi, acc); break;
-      case 5: compute_dir<R, NL, DAG, 2, 1, RB, LS>(a, c, u, psi, acc); break;
-      case 6: compute_dir<R, NL, DAG, 3, 0, RB, LS>(a, c, u, psi, acc); break;
-      default: compute_dir<R, NL, DAG, 3, 1, RB, LS>(a, c, u, psi, acc); break;
-    }
-  }
+    compute_dir<R, NL, DAG, mu, fb, RB, LS>(a, c, u, psi, acc);
+    // the next direction's loads come after these sums
+#pragma unroll
+    for (int j = 0; j < RB; ++j)
+#pragma unroll
+      for (int k = 0; k < 12; ++k) asm volatile("" : "+v"(acc[j][k].x), "+v"(acc[j][k].y));
+    asm volatile("" ::: "memory");
+  };
+  one(std::integral_constant<int, 0>());
+  one(std::integral_constant<int, 1>());
+  one(std::integral_constant<int, 2>());
+  one(std::integral_constant<int, 3>());
+  one(std::integral_constant<int, 4>());
+  one(std::integral_constant<int, 5>());
+  one(std::integral_constant<int, 6>());
+  one(std::integral_constant<int, 7>());
 }
 
 // Visiting order of the 64-site blocks, seg > 1: the bps blocks of a time
@@ -286,6 +294,9 @@ __device__ __forceinline__ long block_order(long T, int seg, int bps, int lt) {
   const long t = off / len;
   return t * bps + lo + (off - t * len);
 }
+
+// entries of a site in the link staging (ls == 1): 72 of links, 36 of clover, a pad
+__host__ __device__ inline int stage_ld(bool clov) { return clov ? 109 : 73; }
 
 // ls == 2 (spinor-block staging) applies to hops of one right-hand side in
 // natural block order whose input is in the working precision, without link
@@ -408,7 +419,8 @@ __global__ __launch_bounds__(512, (hop_min_waves<R, RB>())) void k_hop(const Hop
   };
   // ls: the workgroup's sites v0 .. v0 + ns - 1 get their links, prepared
   // (prepare_link: 9 entries per direction), and the EPI_CLOV blocks (36
-  // entries) copied to LDS once, entry e of site v0 + s at stage[e * ns + s];
+  // entries) copied to LDS once, entry e of site v0 + s at stage[s * ld + e], so
+  // that an item's reads differ by constants, ld odd for its banks;
   // the Gt items of a site then read them from there instead of each loading
   // them through the texture path and preparing the links again
   extern __shared__ __align__(16) char wc_dyn_lds[];
@@ -416,6 +428,7 @@ __global__ __launch_bounds__(512, (hop_min_waves<R, RB>())) void k_hop(const Hop
   const long v0 = Gt == 1 ? q0 : (long)((uint32_t)q0 / (uint32_t)Gt);
   int ns = 0;
   const bool clov_staged = LS && (EPI & EPI_CLOV) && a.clov && !a.clov_roff;
+  const int ld = stage_ld(clov_staged);
   if constexpr (LS) {
     long v1 = (long)((uint32_t)(q0 + (long)blockDim.x - 1) / (uint32_t)Gt);
     if (v1 > g.Vh - 1) v1 = g.Vh - 1;
@@ -431,12 +444,12 @@ __global__ __launch_bounds__(512, (hop_min_waves<R, RB>())) void k_hop(const Hop
       for (int e = 0; e < NL; ++e) u[e] = ((const C *)a.W)[aidx(dir * NL + e, hv, nw)];
       prepare_link<R, NL>(a, dir >> 1, dir & 1, cs, u);
 #pragma unroll
-      for (int e = 0; e < 9; ++e) stage[(dir * 9 + e) * ns + sidx] = u[e];
+      for (int e = 0; e < 9; ++e) stage[sidx * ld + dir * 9 + e] = u[e];
     }
     if (clov_staged)
       for (int i = threadIdx.x; i < 36 * ns; i += blockDim.x) {
         const int e = (int)((uint32_t)i / (uint32_t)ns), sidx = i - e * ns;
-        stage[72 * ns + i] = ((const C *)a.clov)[aidx(e, site_of(v0 + sidx), 36)];
+        stage[sidx * ld + 72 + e] = ((const C *)a.clov)[aidx(e, site_of(v0 + sidx), 36)];
       }
     __syncthreads();
   }
@@ -476,11 +489,11 @@ __global__ __launch_bounds__(512, (hop_min_waves<R, RB>())) void k_hop(const Hop
 #pragma unroll
     for (int k = 0; k < 12; ++k) acc[j][k] = cmk<C>(0, 0);
   hop_site<R, NL, DAG, RB, SI, LS, xs_possible<R, RB, SI, LS>()>(a, h, rb, c[0], c[1], c[2], c[3], acc,
-                                                                   stage + sv, ns, xst, q0, xsn, (int)blockDim.x);
+                                                                   stage + sv * ld, xst, q0, xsn, (int)blockDim.x);
   // epilogue
   const bool zb = a.open_bc && (c[3] == 0 || c[3] == g.L[3] - 1);
   hop_epilogue<R, EPI, RB, SO>(
-      a, h, rb, zb, clov_staged ? stage + 72 * ns + sv : nullptr, (long)ns, acc,
+      a, h, rb, zb, clov_staged ? stage + sv * ld + 72 : nullptr, 1L, acc,
       [&](C y[RB][12]) { load12_rhs<SI, RB>((const SI *)a.y, h, rb, N, y); },
       [&](C dv[RB][12]) { load12_rhs<SI, RB>((const SI *)a.dotv, h, rb, N, dv); });
 }
@@ -508,10 +521,10 @@ static bool hop_epi(const HopLaunch &a, hipStream_t s) {
   // the workgroups per CU at shape.occ
   size_t lds = a.shape.occ > 0 ? (size_t)((kLdsPerCU / a.shape.occ) & ~1023) : 0;
   if (a.shape.ls == 1) {
-    const size_t st = (size_t)(72 + ((a.epi & EPI_CLOV) && a.clov && !a.clov_roff ? 36 : 0)) *
-                      (size_t)stage_sites(threads, G) * sizeof(C);
-    if (st > (size_t)kMaxStageBytes) return false;
-    lds = std::max(lds, st);
+    const bool clov = (a.epi & EPI_CLOV) && a.clov && !a.clov_roff;
+    const size_t st = (size_t)stage_sites(threads, G) * sizeof(C);
+    if ((clov ? 108 : 72) * st > (size_t)kMaxStageBytes) return false;
+    lds = std::max(lds, (size_t)stage_ld(clov) * st);
   } else if (xs_possible<R, RB, SI, false>() && xs_on(a)) {
     const size_t st = (size_t)12 * (size_t)threads * sizeof(C);
     if (st > (size_t)kMaxStageBytes) return false;

@@ -385,7 +385,9 @@ inline wck::HopShape shape_for(const wc_operator *op, int nrhs) {
 // waves as fit are fastest, links staged from 7 right-hand sides on; two and four
 // fill a thread's pairs without a rest.  Normal operator on 24^3 x 48 with
 // 12-real links: 3, 4, 5, 8 and 11 right-hand sides 469, 518, 757, 1010 and 1196
-// us in the FP32 hop's shapes, 430, 491, 645, 785 and 1087 in these.
+// us in the FP32 hop's shapes, 430, 491, 645, 785 and 1087 in these.  From 10 on 8
+// waves share more of what they stage: 12 right-hand sides 1157 us with 4, 1110
+// with 8; 8 right-hand sides 731 and 791.
 inline wck::HopShape default_shape16(const wc_operator *op, int nrhs) {
   wck::HopShape sh;
   if (nrhs <= 2) return default_shape(op, nrhs);
@@ -393,7 +395,7 @@ inline wck::HopShape default_shape16(const wc_operator *op, int nrhs) {
     sh.rb = 2;
     return sh;
   }
-  sh.tpb = widest(op->g.Vh / kBlk * nrhs, 4);
+  sh.tpb = widest(op->g.Vh / kBlk * nrhs, nrhs >= 10 ? 8 : 4);
   sh.ls = nrhs >= 7 ? 1 : 0;
   if (!stage_fits(op, nrhs, sh)) sh.ls = 0;
   return sh;

@@ -435,9 +435,12 @@ class site_scalar:
 
 
 def plain(t, dtype):
-    """whether a kernel can take the values of t as they lie in memory"""
+    """whether a kernel on the current device can take the values of t as they lie
+    in memory, and nothing is differentiated"""
     return (t.dtype == dtype and t.is_contiguous() and t.device == device()
-            and not (t.is_conj() or t.is_neg() or t.requires_grad))
+            and t.device.index == torch.cuda.current_device()
+            and not (t.is_conj() or t.is_neg() or t.requires_grad)
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
 
 
 def trace(x):

@@ -109,14 +109,17 @@ static int build_own_clover(wc_operator *op, hipStream_t s) {
   return WC_OK;
 }
 
-// whether a kernel can read p: device (or managed) memory
+// whether a kernel on the current device can read p: its own memory, or managed
+// memory (another device's may not be mapped here)
 static bool on_device(const void *p) {
   hipPointerAttribute_t at{};
   if (hipPointerGetAttributes(&at, p) != hipSuccess) {
     (void)hipGetLastError();  // host memory that HIP does not know
     return false;
   }
-  return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  return (at.type == hipMemoryTypeDevice && at.device == dev) || at.type == hipMemoryTypeManaged;
 }
 
 // links and clover from four natural link fields; one that a kernel cannot

@@ -80,3 +80,17 @@ def test_infinities_stay_in_their_slice():
     got = g.slice(g.trace(a * g.adj(a)), 3)
     assert got[3].real == float("inf") or np.isnan(got[3].real)
     assert [x for t, x in enumerate(got) if t != 3] == [x for t, x in enumerate(fin) if t != 3]
+
+
+def test_derivatives_take_the_general_path():
+    grid = g.grid([4, 4, 4, 4], g.double)
+    a, b = prop(grid, 1), prop(grid, 2)
+    want = g.trace(b * g.adj(b)).data
+    p, t = a.data.clone(), b.data
+    with torch.autograd.forward_ad.dual_level():
+        a.data = torch.autograd.forward_ad.make_dual(p, t)
+        tangent = torch.autograd.forward_ad.unpack_dual(g.trace(a * g.adj(b)).data).tangent
+    assert float((tangent - want).abs().max()) < 1e-12 * float(want.abs().max())
+    a.data = p.requires_grad_(True)
+    g.trace(a * g.adj(b)).data.real.sum().backward()
+    assert torch.equal(p.grad, b.data)

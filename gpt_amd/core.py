@@ -434,10 +434,19 @@ class site_scalar:
         return self.data.cpu().numpy().reshape(tuple(reversed(self.grid.fdimensions)))
 
 
+def eager():
+    """whether torch runs the calls as they stand.  A kernel is no operation of
+    torch's: a trace (make_fx, jit, compile) would lack it, a dispatch mode not see
+    it, and a tensor under a transform (vmap, jvp, ...) has no address to give it"""
+    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+                or torch._C._get_tracing_state() is not None
+                or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def plain(t, dtype):
     """whether a kernel on the current device can take the values of t as they lie
-    in memory, and nothing is differentiated"""
-    return (t.dtype == dtype and t.is_contiguous() and t.device == device()
+    in memory, and nothing is differentiated (where calls are eager)"""
+    return (type(t) is torch.Tensor and t.dtype == dtype and t.is_contiguous() and t.device == device()
             and t.device.index == torch.cuda.current_device()
             and not (t.is_conj() or t.is_neg() or t.requires_grad)
             and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
@@ -450,7 +459,8 @@ def trace(x):
     if isinstance(x, _site_product):
         a, b = x.a.data, x.b.data
         prec = {torch.complex128: double, torch.complex64: single}.get(a.dtype)
-        if prec is not None and a.shape == b.shape and a[0].numel() == 144 and plain(a, a.dtype) and plain(b, a.dtype):
+        if (prec is not None and eager() and a.shape == b.shape and a[0].numel() == 144 and plain(a, a.dtype)
+                and plain(b, a.dtype)):
             out = torch.empty(a.shape[0], dtype=torch.complex128, device=a.device)
             _lib.check(_lib.load().wc_site_trace(prec.code, a.shape[0], a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                                  stream_ptr()))
@@ -471,7 +481,7 @@ def slice_(x, dim):
     L = x.grid.fdimensions
     inner = int(np.prod(L[:dim])) if 0 <= dim < 4 else 0
     # runs of less than 128 bytes (slices in x) are left to the general sum
-    if inner >= 8 and x.data.numel() == int(np.prod(L)) and plain(x.data, torch.complex128):
+    if inner >= 8 and eager() and x.data.numel() == int(np.prod(L)) and plain(x.data, torch.complex128):
         n = L[dim]
         work = torch.empty((17, n), dtype=torch.complex128, device=x.data.device)
         _lib.check(_lib.load().wc_slice_sum(x.data.numel() // (n * inner), n, inner, x.data.data_ptr(),

@@ -519,7 +519,7 @@ def _pointers(fields, packed, written):
     are written, apart from each other and from it"""
     t = packed.data
     shape = t.shape[:-2] + (1, 2)
-    if len(fields) < 2 or not core.plain(t, t.dtype):
+    if len(fields) < 2 or not core.eager() or not core.plain(t, t.dtype):
         return None
     if not all(f.data.shape == shape and core.plain(f.data, t.dtype) for f in fields):
         return None

@@ -446,7 +446,7 @@ def eager():
 def plain(t, dtype):
     """whether a kernel on the current device can take the values of t as they lie
     in memory, and nothing is differentiated (where calls are eager)"""
-    return (type(t) is torch.Tensor and t.dtype == dtype and t.is_contiguous() and t.device == device()
+    return (type(t) is torch.Tensor and t.is_cuda and t.dtype == dtype and t.is_contiguous() and t.device == device()
             and t.device.index == torch.cuda.current_device()
             and not (t.is_conj() or t.is_neg() or t.requires_grad)
             and torch.autograd.forward_ad.unpack_dual(t).tangent is None)

@@ -1,0 +1,35 @@
+"""g.trace and g.slice of values that lie in host memory, on a machine without a
+GPU too, and directions given as other numbers than int: against numpy."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import gpt_amd as g  # noqa: E402
+from gpt_amd import core  # noqa: E402
+
+GRID = g.grid([4, 6, 8, 4], g.double)
+
+
+def host_field(seed, prec=g.double):
+    p = core.mspincolor_lattice.__new__(core.mspincolor_lattice)
+    p.grid = g.grid(GRID.fdimensions, prec)
+    rng = np.random.default_rng(seed)
+    a = rng.standard_normal((GRID.gsites, 4, 4, 3, 3)) + 1j * rng.standard_normal((GRID.gsites, 4, 4, 3, 3))
+    p.data = torch.from_numpy(a.astype(prec.complex_dtype))
+    return p
+
+
+@pytest.mark.parametrize("prec", [g.double, g.single], ids=["double", "single"])
+def test_values_in_host_memory(prec):
+    a, b = host_field(1, prec), host_field(2, prec)
+    x, y = (p.data.numpy().astype(np.complex128).reshape(GRID.gsites, -1) for p in (a, b))
+    want = (x * y.conj()).sum(1)
+    # 144 products and sums of numbers of order 1
+    assert np.abs(g.trace(a * g.adj(b)).data.numpy() - want).max() <= 148 * 2.3e-16 * 40
+    tr = core.site_scalar(GRID, torch.from_numpy(want))
+    f = want.reshape(GRID.fdimensions[::-1])
+    for dim in range(4):
+        other = tuple(d for d in range(4) if d != 3 - dim)
+        ref = f.sum(other)
+        assert np.abs(np.array(g.slice(tr, dim)) - ref).max() <= f.size * 2.3e-16 * np.abs(f).max()

@@ -479,7 +479,7 @@ def slice_(x, dim):
     if not isinstance(x, site_scalar):
         raise NotImplementedError("g.slice is provided for g.trace results")
     L = x.grid.fdimensions
-    inner = int(np.prod(L[:dim])) if 0 <= dim < 4 else 0
+    inner = int(np.prod(L[:dim])) if isinstance(dim, numbers.Integral) and 0 <= dim < 4 else 0
     # runs of less than 128 bytes (slices in x) are left to the general sum
     if inner >= 8 and eager() and x.data.numel() == int(np.prod(L)) and plain(x.data, torch.complex128):
         n = L[dim]

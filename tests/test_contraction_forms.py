@@ -33,3 +33,14 @@ def test_values_in_host_memory(prec):
         other = tuple(d for d in range(4) if d != 3 - dim)
         ref = f.sum(other)
         assert np.abs(np.array(g.slice(tr, dim)) - ref).max() <= f.size * 2.3e-16 * np.abs(f).max()
+
+
+@pytest.mark.parametrize("kind", [float, np.float64, np.int64, np.uint8, torch.tensor], ids=lambda k: k.__name__)
+def test_directions_as_other_numbers(kind):
+    rng = np.random.default_rng(3)
+    tr = core.site_scalar(GRID, torch.from_numpy(rng.standard_normal(GRID.gsites) + 0j))
+    for dim in range(4):
+        assert g.slice(tr, kind(dim)) == g.slice(tr, dim)
+    for dim in (4, -1):
+        with pytest.raises(TypeError):
+            g.slice(tr, kind(dim) if kind is not np.uint8 else 4)

@@ -553,7 +553,7 @@ def unpack(field, dst=None):
         dst = [lattice(field.grid.single_rhs()) for _ in range(n)]
         for x in dst:
             x._cb = field.checkerboard()
-    ptrs = _pointers(dst[:n], field, True) if len(dst) >= n else None
+    ptrs = _pointers([dst[r] for r in range(n)], field, True)
     if ptrs is not None:
         _lib.check(_lib.load().wc_unpack_rhs(field.grid.precision.code, field.nentries // n, n, field.ptr(), ptrs,
                                              core.stream_ptr()))

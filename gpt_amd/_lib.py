@@ -75,6 +75,8 @@ SIGNATURES = {
     "wc_tune_hop": (_I, [_P, _I, _I, _P, _P, _P]),
     "wc_set_hop_shape": (_I, [_P, _I, _P]),
     "wc_get_hop_shape": (_I, [_P, _I, _P]),
+    "wc_set_hop_form": (_I, [_P, _I, _I]),
+    "wc_get_hop_form": (_I, [_P, _I, _P]),
     "wc_set_iteration_chunk": (_I, [_P, _I]),
     "wc_trim": (_I, [_P]),
     "wc_release_cached_memory": (_I, [_P]),

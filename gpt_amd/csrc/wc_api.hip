@@ -1077,6 +1077,13 @@ int maybe_tune(wc_operator *op, int nrhs, hipStream_t s) {
   return rc;
 }
 
+// the form that the hop takes
+template <typename R> static int form_taken(const wc_operator *op, int nrhs) {
+  const HopLaunch a = hop_args<R>(op, nrhs, 0, 0, 0, nullptr, nullptr);
+  if (wck::hop_split_applies<R>(a)) return WC_HOP_FORM_SPLIT;
+  return wck::hop_march_applies<R>(a) ? WC_HOP_FORM_MARCH : WC_HOP_FORM_GATHER;
+}
+
 extern "C" {
 
 int wc_tune_hop(wc_operator *op, int nrhs, int reps, int *shape, float *ms_per_call, void *stream) {
@@ -1131,6 +1138,22 @@ int wc_get_hop_shape(const wc_operator *op, int nrhs, int *shape) {
   shape[2] = sh.occ;
   shape[3] = sh.seg;
   shape[4] = sh.ls;
+  return WC_OK;
+}
+
+int wc_set_hop_form(wc_operator *op, int nrhs, int form) {
+  if (!op) WC_FAIL(WC_ERR_ARG, "wc_set_hop_form: null operator");
+  if (nrhs < 1 || nrhs > 64) WC_FAIL(WC_ERR_ARG, "wc_set_hop_form: nrhs = %d must be in [1, 64]", nrhs);
+  if (form < WC_HOP_FORM_DEFAULT || form > WC_HOP_FORM_SPLIT)
+    WC_FAIL(WC_ERR_ARG, "wc_set_hop_form: form %d is not in [%d, %d]", form, WC_HOP_FORM_DEFAULT, WC_HOP_FORM_SPLIT);
+  op->form[nrhs] = form;
+  return WC_OK;
+}
+
+int wc_get_hop_form(const wc_operator *op, int nrhs, int *form) {
+  if (!op || !form) WC_FAIL(WC_ERR_ARG, "wc_get_hop_form: null argument");
+  if (nrhs < 1 || nrhs > 64) WC_FAIL(WC_ERR_ARG, "wc_get_hop_form: nrhs = %d must be in [1, 64]", nrhs);
+  *form = op->prec == WC_DOUBLE ? form_taken<double>(op, nrhs) : form_taken<float>(op, nrhs);
   return WC_OK;
 }
 

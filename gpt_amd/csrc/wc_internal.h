@@ -159,6 +159,7 @@ struct wc_operator {
   wck::HopShape shape[65];      // hop launch shape per right-hand-side count
   bool shape_set[65] = {};      // shape chosen (by the tuner or the caller)
   bool shape_user[65] = {};     // shape set by the caller (wc_set_hop_shape): used for 16-bit hops too
+  int form[65] = {};            // the hop's form (WC_HOP_FORM_*) as the caller set it
   int chunk = 0;                // iterations per run: 0 automatic, 1 one at a time, else at most this many
   // FP16-storage hops of 4k right-hand sides: 0 vector ALUs, 1 matrix cores,
   // 2 automatic (the faster of the two, timed per lattice and class of
@@ -436,6 +437,14 @@ inline int mma_for(const wc_operator *op, int nrhs) {
 int build_mass_blocks(const wc_operator *op, double mass, void *ai0, void *ai1, void *a0, void *a1, int *err,
                       hipStream_t s);
 
+// the forms that a hop may take: the caller's, else all of them, else (a shape
+// set by hand is for the gathering kernel) that one
+inline int form_for(const wc_operator *op, int nrhs) {
+  if (nrhs < 1 || nrhs > 64) return WC_HOP_FORM_AUTO;
+  if (op->form[nrhs] != WC_HOP_FORM_DEFAULT) return op->form[nrhs];
+  return op->shape_user[nrhs] ? WC_HOP_FORM_GATHER : WC_HOP_FORM_AUTO;
+}
+
 // ------------------------------------------------------------ compositions
 template <typename R>
 inline HopLaunch hop_args(const wc_operator *op, int nrhs, int pout, int dag, int epi, const void *in, void *out) {
@@ -463,10 +472,9 @@ inline HopLaunch hop_args(const wc_operator *op, int nrhs, int pout, int dag, in
   a.halt = op->halt_cur;
   a.mma = mma_for(op, nrhs);
   a.clov_roff = clov_roff(op);
-  // a caller's shape is for the gathering kernel
-  const bool user = nrhs >= 1 && nrhs <= 64 && op->shape_user[nrhs];
-  a.split = user ? 0 : 1;
-  a.march = user || a.shape.form == 2 ? 0 : a.shape.form == 1 ? 1 : 2;
+  const int f = form_for(op, nrhs);
+  a.split = f == WC_HOP_FORM_AUTO || f == WC_HOP_FORM_SPLIT ? 1 : 0;
+  a.march = f == WC_HOP_FORM_MARCH ? 1 : f != WC_HOP_FORM_AUTO || a.shape.form == 2 ? 0 : a.shape.form == 1 ? 1 : 2;
   return a;
 }
 
@@ -643,7 +651,7 @@ inline void op_key(const wc_operator *op, int nrhs, std::vector<uintptr_t> &key)
                       (uintptr_t)clov_inv(op, 1), (uintptr_t)clov_roff(op), tmp(0), tmp(1), tmp(2), (uintptr_t)op->dots, (uintptr_t)op->partials, bits(op->diag), bits(op->cs), bits(op->ct), (uintptr_t)op->open_bc,
                       (uintptr_t)op->has_clover, (uintptr_t)sh.rb, (uintptr_t)sh.tpb, (uintptr_t)sh.occ,
                       (uintptr_t)sh.seg, (uintptr_t)sh.ls, (uintptr_t)op->bps, (uintptr_t)s16.rb, (uintptr_t)s16.tpb,
-                      (uintptr_t)s16.occ, (uintptr_t)s16.seg, (uintptr_t)s16.ls, (uintptr_t)mma_for(op, nrhs), (uintptr_t)op->shape_user[nrhs], (uintptr_t)sh.form})
+                      (uintptr_t)s16.occ, (uintptr_t)s16.seg, (uintptr_t)s16.ls, (uintptr_t)mma_for(op, nrhs), (uintptr_t)form_for(op, nrhs), (uintptr_t)sh.form})
     key.push_back(v);
   for (int mu = 0; mu < 4; ++mu) {
     key.push_back(bits(op->p.boundary_phases[mu][0]));

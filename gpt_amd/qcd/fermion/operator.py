@@ -30,6 +30,9 @@ OPCODES = {
 }
 FULL_FIELD = {2001, 2002, 2009, 2010, 2011, 2012, 2013, 2014, 2015, 3001, 4001}
 
+# codes of the hop's forms (WC_HOP_FORM_*)
+HOP_FORMS = (None, "auto", "gather", "march", "split")
+
 # pool of suspended operator handles by tag (interface.py:23-24)
 operator_tag = {}
 operator_limbo = {}
@@ -265,13 +268,30 @@ class fine_operator(matrix_operator):
         return tuple(sh)
 
     def set_hop_shape(self, shape, n_rhs=None):
-        """shape = (rb, tpb, occ, seg, ls), or None for automatic"""
+        """shape = (rb, tpb, occ, seg, ls), or None for automatic.  Without
+        set_hop_form, a shape (also one that hop_shape or tune_hop gave) selects
+        the gathering kernel"""
         n = self.n_rhs if n_rhs is None else int(n_rhs)
         if shape is None:
             _lib.check(_lib.load().wc_set_hop_shape(self.handle, n, None))
             return
         sh = (ctypes.c_int * 5)(*[int(x) for x in shape])
         _lib.check(_lib.load().wc_set_hop_shape(self.handle, n, ctypes.addressof(sh)))
+
+    # the hop's form (wc_set_hop_form): "auto" (by size and measurement, beside a
+    # shape set by hand too), "gather", "march" (through t; many right-hand sides)
+    # or "split" (one wave per direction; few sites), or None, the default: "auto",
+    # and "gather" where a shape is set by hand.  Bitwise the same results
+    def set_hop_form(self, form, n_rhs=None):
+        n = self.n_rhs if n_rhs is None else int(n_rhs)
+        _lib.check(_lib.load().wc_set_hop_form(self.handle, n, HOP_FORMS.index(form)))
+
+    def hop_form(self, n_rhs=None):
+        """the form that Meooe of n_rhs right-hand sides takes now"""
+        n = self.n_rhs if n_rhs is None else int(n_rhs)
+        f = ctypes.c_int()
+        _lib.check(_lib.load().wc_get_hop_form(self.handle, n, ctypes.byref(f)))
+        return HOP_FORMS[f.value]
 
     # FP16-storage hops of 4k right-hand sides on the matrix cores
     # (wc_set_hop_mma): True, False, or "auto" (the default: the faster form,

@@ -252,10 +252,33 @@ int wc_solve_eo2_ne_block_cg(wc_operator *op, int parity, int nrhs, void *dst, c
  * The CG, solve and batch entry points tune on first use when
  * Vh * nrhs >= 2^17, once per class (environment WC_AUTOTUNE=0 turns tuning
  * off).  The tuner leaves seg at 1.  wc_set_hop_shape fixes a shape (NULL:
- * back to automatic); wc_get_hop_shape reports the one in use. */
+ * back to automatic); wc_get_hop_shape reports the one in use.
+ *
+ * A shape is the gathering kernel's, one of the three forms below.  By default
+ * (WC_HOP_FORM_DEFAULT) a hop in the operator's own precision takes the form that
+ * its size and the tuner's measurement give, whatever its shape; but a shape
+ * fixed by wc_set_hop_shape, also one that wc_tune_hop or wc_get_hop_shape has
+ * just reported, is a choice of the gathering kernel.  wc_set_hop_form
+ * says otherwise, and holds until it is called again, whatever shapes are set:
+ *   WC_HOP_FORM_AUTO    by size and measurement, beside a fixed shape too;
+ *   WC_HOP_FORM_GATHER  the gathering kernel;
+ *   WC_HOP_FORM_MARCH   waves that walk through t (8, or 10 and more, right-hand
+ *                       sides in FP64, 7 and more in FP32);
+ *   WC_HOP_FORM_SPLIT   one wave per direction (at most 16384 pairs of site and
+ *                       right-hand side in FP64, 32768 in FP32).
+ * Hops that do not have the form set take the gathering kernel.
+ * wc_get_hop_form reports the one that Meooe of nrhs right-hand sides takes
+ * now (GATHER, MARCH or SPLIT).  All forms give bitwise the same result. */
+#define WC_HOP_FORM_DEFAULT 0
+#define WC_HOP_FORM_AUTO 1
+#define WC_HOP_FORM_GATHER 2
+#define WC_HOP_FORM_MARCH 3
+#define WC_HOP_FORM_SPLIT 4
 int wc_tune_hop(wc_operator *op, int nrhs, int reps, int *shape, float *ms_per_call, void *stream);
 int wc_set_hop_shape(wc_operator *op, int nrhs, const int *shape);
 int wc_get_hop_shape(const wc_operator *op, int nrhs, int *shape);
+int wc_set_hop_form(wc_operator *op, int nrhs, int form);
+int wc_get_hop_form(const wc_operator *op, int nrhs, int *form);
 
 /* Matrix cores for the FP16-storage hops (no cgpt counterpart: Grid's 5-d
  * multi-RHS operator, lib/cgpt/lib/operators/wilson_clover.h:58-66, runs its

@@ -36,6 +36,8 @@ HOP_FORMS = (None, "auto", "gather", "march", "split")
 # pool of suspended operator handles by tag (interface.py:23-24)
 operator_tag = {}
 operator_limbo = {}
+# the right-hand-side counts whose launch shape or form was set by hand, by handle
+operator_shaped = {}
 
 
 def release_pool():
@@ -46,6 +48,7 @@ def release_pool():
         while handles:
             h = handles.pop()
             operator_tag.pop(h, None)
+            operator_shaped.pop(h, None)
             _lib.check(_lib.load().wc_destroy(h))
             n += 1
     return n
@@ -71,6 +74,7 @@ class interface:
 
     def __init__(self):
         self.obj = None
+        self.shaped = None  # the parked handle's entry of operator_shaped
 
     def _setup(self, grid, params, U):
         assert self.obj is None
@@ -85,7 +89,12 @@ class interface:
             _lib.check(lib.wc_set_mass(self.obj, float(params["mass"]), stream))
             _lib.check(lib.wc_update(self.obj, Ut.data_ptr(), stream))
             _lib.check(lib.wc_set_iteration_chunk(self.obj, 0))  # a new operator's default schedule
-            _lib.check(lib.wc_set_hop_mma(self.obj, 2))  # and its default (automatic) hop form
+            _lib.check(lib.wc_set_hop_mma(self.obj, 2))  # its default (automatic) hop form
+            # and, where another owner had set others, the automatic launch shapes and forms
+            if operator_shaped.get(self.obj) is not self.shaped:
+                for n in operator_shaped.pop(self.obj, ()):
+                    _lib.check(lib.wc_set_hop_shape(self.obj, n, None))
+                    _lib.check(lib.wc_set_hop_form(self.obj, n, HOP_FORMS.index(None)))
         else:
             p = _lib.wc_params()
             for i in range(4):
@@ -124,6 +133,7 @@ class interface:
                 _lib.check(_lib.load().wc_trim(self.obj))
             except Exception:  # interpreter shutdown: the runtime may be gone
                 pass
+            self.shaped = operator_shaped.get(self.obj)
             operator_limbo.setdefault(operator_tag[self.obj], []).append(self.obj)
             self.obj = None
 
@@ -131,6 +141,7 @@ class interface:
         """free the native operator now instead of parking it in the pool"""
         if self.obj is not None:
             operator_tag.pop(self.obj, None)
+            operator_shaped.pop(self.obj, None)
             _lib.check(_lib.load().wc_destroy(self.obj))
             self.obj = None
 
@@ -277,6 +288,7 @@ class fine_operator(matrix_operator):
             return
         sh = (ctypes.c_int * 5)(*[int(x) for x in shape])
         _lib.check(_lib.load().wc_set_hop_shape(self.handle, n, ctypes.addressof(sh)))
+        operator_shaped.setdefault(self.handle, set()).add(n)
 
     # the hop's form (wc_set_hop_form): "auto" (by size and measurement, beside a
     # shape set by hand too), "gather", "march" (through t; many right-hand sides)
@@ -285,6 +297,7 @@ class fine_operator(matrix_operator):
     def set_hop_form(self, form, n_rhs=None):
         n = self.n_rhs if n_rhs is None else int(n_rhs)
         _lib.check(_lib.load().wc_set_hop_form(self.handle, n, HOP_FORMS.index(form)))
+        operator_shaped.setdefault(self.handle, set()).add(n)
 
     def hop_form(self, n_rhs=None):
         """the form that Meooe of n_rhs right-hand sides takes now"""

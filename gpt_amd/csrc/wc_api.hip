@@ -687,8 +687,20 @@ static int mixed_impl(wc_operator *hi, wc_operator *lo, int N, int pd, void *dst
 }
 
 // ------------------------------------------------------------- hop tuner
+// the form that the hop takes
+template <typename R> static int form_taken(const wc_operator *op, int nrhs) {
+  const HopLaunch a = hop_args<R>(op, nrhs, 0, 0, 0, nullptr, nullptr);
+  if (wck::hop_split_applies<R>(a)) return WC_HOP_FORM_SPLIT;
+  return wck::hop_march_applies<R>(a) ? WC_HOP_FORM_MARCH : WC_HOP_FORM_GATHER;
+}
+static int form_taken(const wc_operator *op, int nrhs) {
+  return op->prec == WC_DOUBLE ? form_taken<double>(op, nrhs) : form_taken<float>(op, nrhs);
+}
+
 // Times the hop (output parity 0, clover epilogue) of nrhs right-hand sides
-// for every valid launch shape and returns the fastest.  Scratch: tmp[0..1];
+// for every valid launch shape and returns the fastest.  A hop that takes
+// one wave per direction has no shapes: its time is returned with the one in
+// use.  Scratch: tmp[0..1];
 // the input is a fixed pattern of values in [-1, 1) (no denormals or NaN,
 // and not zero: all-zero input runs faster, by an amount that depends on the
 // shape), the output is overwritten.
@@ -705,7 +717,9 @@ static int tune_impl(wc_operator *op, int N, int reps, hipStream_t s, wck::HopSh
   // right-hand side; the t-marching order (seg > 1) is tried second, on the
   // fastest shape in natural order
   const int occs[] = {0, 2, 4, 8, 16};
-  for (int rb = 1; rb <= max_rb_prec(op->prec) && rb <= N; ++rb)
+  const int split = form_taken<R>(op, N) == WC_HOP_FORM_SPLIT;
+  if (split) cand.push_back(shape_for(op, N));
+  for (int rb = 1; !split && rb <= max_rb_prec(op->prec) && rb <= N; ++rb)
     for (int ls = 0; ls <= 2; ++ls)
       for (int tpb = 1; tpb <= wck::kMaxTpb; tpb *= 2)
         for (int oc : occs) {
@@ -728,7 +742,7 @@ static int tune_impl(wc_operator *op, int N, int reps, hipStream_t s, wck::HopSh
     HopLaunch a = hop_args<R>(op, N, 0, 0, op->has_clover ? wck::EPI_CLOV : 0, op->tmp[0], op->tmp[1]);
     a.clov = op->has_clover ? op->Ai[0] : nullptr;
     a.shape = sh;
-    a.split = 0;
+    a.split = split;
     a.march = march;
     // shapes this device cannot launch, or whose staging area is too large
     if (!wck::hop<R>(a, s) || hipGetLastError() != hipSuccess) return WC_OK;
@@ -752,7 +766,7 @@ static int tune_impl(wc_operator *op, int N, int reps, hipStream_t s, wck::HopSh
   // 4 runs per slice, 11 % faster than natural order).  The natural-order
   // winner is timed again beside its t-marching variants: its first time is
   // the minimum over many noisy candidates and would be biased low.
-  if (!rc && best_ms >= 0.0f && best.ls != 2 && op->bps > 1) {
+  if (!rc && !split && best_ms >= 0.0f && best.ls != 2 && op->bps > 1) {
     const wck::HopShape nat = best;
     best_ms = -1.0f;
     rc = try_shape(nat);
@@ -771,7 +785,7 @@ static int tune_impl(wc_operator *op, int N, int reps, hipStream_t s, wck::HopSh
   // compared (with and without the clover), the better of three rounds in turn:
   // by that one hop and one round, 16^3 x 32 (Mpc^dag Mpc 330 us against 360) now
   // and then took the slower form.
-  if (!rc && best_ms >= 0.0f) {
+  if (!rc && !split && best_ms >= 0.0f) {
     HopLaunch a = hop_args<R>(op, N, 0, 0, op->has_clover ? wck::EPI_CLOV : 0, op->tmp[0], op->tmp[1]);
     a.clov = op->has_clover ? op->Ai[0] : nullptr;
     a.march = 1;
@@ -923,12 +937,21 @@ static std::string s16_tag(const wc_operator *op, int nrhs, bool try_mma) {
 static int tune_hop(wc_operator *op, int nrhs, int reps, hipStream_t s, float *ms_out) {
   wck::HopShape best;
   float ms = 0.0f;
+  const bool set = op->shape_set[nrhs], user = op->shape_user[nrhs];
+  if (user) op->shape_set[nrhs] = op->shape_user[nrhs] = false;  // a caller's shape ends here
   int rc = op->prec == WC_DOUBLE ? tune_impl<double>(op, nrhs, reps, s, best, ms)
                                  : tune_impl<float>(op, nrhs, reps, s, best, ms);
-  if (rc) return rc;
+  if (rc) {
+    op->shape_set[nrhs] = set;
+    op->shape_user[nrhs] = user;
+    return rc;
+  }
+  if (form_taken(op, nrhs) == WC_HOP_FORM_SPLIT) {  // no shape was chosen
+    if (ms_out) *ms_out = ms;
+    return WC_OK;
+  }
   op->shape[nrhs] = best;
   op->shape_set[nrhs] = true;
-  op->shape_user[nrhs] = false;
   {
     std::lock_guard<std::mutex> lk(g_shape_mu);
     g_shape_cache[shape_key(op, nrhs)] = best;
@@ -1077,13 +1100,6 @@ int maybe_tune(wc_operator *op, int nrhs, hipStream_t s) {
   return rc;
 }
 
-// the form that the hop takes
-template <typename R> static int form_taken(const wc_operator *op, int nrhs) {
-  const HopLaunch a = hop_args<R>(op, nrhs, 0, 0, 0, nullptr, nullptr);
-  if (wck::hop_split_applies<R>(a)) return WC_HOP_FORM_SPLIT;
-  return wck::hop_march_applies<R>(a) ? WC_HOP_FORM_MARCH : WC_HOP_FORM_GATHER;
-}
-
 extern "C" {
 
 int wc_tune_hop(wc_operator *op, int nrhs, int reps, int *shape, float *ms_per_call, void *stream) {
@@ -1092,14 +1108,7 @@ int wc_tune_hop(wc_operator *op, int nrhs, int reps, int *shape, float *ms_per_c
   if (rc) return rc;
   if (reps < 1) WC_FAIL(WC_ERR_ARG, "wc_tune_hop: reps must be >= 1");
   if ((rc = tune_hop(op, nrhs, reps, (hipStream_t)stream, ms_per_call))) return rc;
-  if (shape) {
-    shape[0] = op->shape[nrhs].rb;
-    shape[1] = op->shape[nrhs].tpb;
-    shape[2] = op->shape[nrhs].occ;
-    shape[3] = op->shape[nrhs].seg;
-    shape[4] = op->shape[nrhs].ls;
-  }
-  return WC_OK;
+  return shape ? wc_get_hop_shape(op, nrhs, shape) : WC_OK;
 }
 
 int wc_set_hop_shape(wc_operator *op, int nrhs, const int *shape) {
@@ -1153,7 +1162,7 @@ int wc_set_hop_form(wc_operator *op, int nrhs, int form) {
 int wc_get_hop_form(const wc_operator *op, int nrhs, int *form) {
   if (!op || !form) WC_FAIL(WC_ERR_ARG, "wc_get_hop_form: null argument");
   if (nrhs < 1 || nrhs > 64) WC_FAIL(WC_ERR_ARG, "wc_get_hop_form: nrhs = %d must be in [1, 64]", nrhs);
-  *form = op->prec == WC_DOUBLE ? form_taken<double>(op, nrhs) : form_taken<float>(op, nrhs);
+  *form = form_taken(op, nrhs);
   return WC_OK;
 }
 

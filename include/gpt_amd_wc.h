@@ -251,8 +251,10 @@ int wc_solve_eo2_ne_block_cg(wc_operator *op, int parity, int nrhs, void *dst, c
  * 4-7, 8-15, 16-31, 32-64).  shape (5 ints) and ms_per_call may be NULL.
  * The CG, solve and batch entry points tune on first use when
  * Vh * nrhs >= 2^17, once per class (environment WC_AUTOTUNE=0 turns tuning
- * off).  The tuner leaves seg at 1.  wc_set_hop_shape fixes a shape (NULL:
- * back to automatic); wc_get_hop_shape reports the one in use.
+ * off).  Where the hop takes the SPLIT form below there is no shape to
+ * choose: its time is returned, and shape is the one already there.
+ * wc_set_hop_shape fixes a shape (NULL: back to automatic); wc_get_hop_shape
+ * reports the one in use.
  *
  * A shape is the gathering kernel's, one of the three forms below.  By default
  * (WC_HOP_FORM_DEFAULT) a hop in the operator's own precision takes the form that

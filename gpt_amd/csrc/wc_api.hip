@@ -830,7 +830,7 @@ static int tune_impl(wc_operator *op, int N, int reps, hipStream_t s, wck::HopSh
 // object, .gpt_auto_tune/<sha256(tag)>.json in the working directory, written
 // after tuning and read when the object is set up
 // (lib/gpt/core/auto_tune.py:20-37,99-136).  The hop tuner does the same:
-// one file per (device, lattice, precision, link format, class of
+// one file per (kernels, device, lattice, precision, link format, class of
 // right-hand-side counts) in the directory WC_TUNE_CACHE (default
 // .gpt_amd_auto_tune; empty or 0: nothing read or written), holding
 // {"tag": ..., "params": [rb, tpb, occ, seg, ls], "ms": ...}.  A shape read
@@ -843,8 +843,12 @@ static std::string tune_cache_dir() {
   return e;
 }
 
-// tag and file name: device architecture and CU count, lattice, precision,
-// link format, right-hand-side class
+// tag and file name: the kernels that were timed, device architecture and CU
+// count, lattice, precision, link format, right-hand-side class.  kTimedKernels
+// changes whenever the hop's kernels or what the tuner times do: a shape picked
+// for others is no measurement of these.  (1: without the marching and the
+// one-wave-per-direction form, timed on an input of zeros.)
+constexpr int kTimedKernels = 2;
 static std::string tune_tag(const wc_operator *op, int nrhs) {
   int dev = 0;
   hipDeviceProp_t pr{};
@@ -856,8 +860,8 @@ static std::string tune_tag(const wc_operator *op, int nrhs) {
     cus = pr.multiProcessorCount;
   }
   char b[256];
-  snprintf(b, sizeof b, "hop_%s_cu%d_%dx%dx%dx%d_%s_links%d_rhs%d", arch.c_str(), cus, op->g.L[0], op->g.L[1],
-           op->g.L[2], op->g.L[3], op->prec == WC_DOUBLE ? "f64" : "f32", 2 * op->nl, nrhs_class(nrhs));
+  snprintf(b, sizeof b, "hop%d_%s_cu%d_%dx%dx%dx%d_%s_links%d_rhs%d", kTimedKernels, arch.c_str(), cus, op->g.L[0],
+           op->g.L[1], op->g.L[2], op->g.L[3], op->prec == WC_DOUBLE ? "f64" : "f32", 2 * op->nl, nrhs_class(nrhs));
   std::string t = b;
   for (char &c : t)
     if (!isalnum((unsigned char)c) && c != '_' && c != '-') c = '_';

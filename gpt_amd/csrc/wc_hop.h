@@ -391,6 +391,12 @@ __device__ __forceinline__ void hop_epilogue(const HopLaunch &a, long h, int rb,
 // with one right-hand side per thread (<= 128 VGPRs), else 2 (<= 256; keeps
 // the compiler from parking accumulators in AGPRs at 1 wave)
 template <typename R, int RB> constexpr int hop_min_waves() { return (sizeof(R) == 4 && RB == 1) ? 4 : 2; }
+// and the most: in FP64 two, whatever registers a kernel gets by with.  The
+// sites in flight decide how often an input spinor is fetched again, and a third
+// wave, which the bare and the axpy hop with staged links have registers for
+// (158), cost more than it hid: Meooe of 9 right-hand sides 24^3 x 48 690 us with
+// three, 607 with two; 6 on 28^3 x 56 819 and 712.
+template <typename R> constexpr int hop_max_waves() { return sizeof(R) == 8 ? 2 : 8; }
 
 // Work items are (site h, right-hand-side group g) with g fastest, g covering
 // the RB right-hand sides g*RB .. g*RB+RB-1, one item per thread over the
@@ -401,7 +407,9 @@ template <typename R, int RB> constexpr int hop_min_waves() { return (sizeof(R) 
 // sums them per 64-site block in site order, so the sums do not depend on
 // the launch shape.
 template <typename R, int NL, int DAG, int EPI, int RB, typename SI, typename SO, bool LS>
-__global__ __launch_bounds__(512, (hop_min_waves<R, RB>())) void k_hop(const HopLaunch a) {
+__global__ __attribute__((amdgpu_flat_work_group_size(1, 512),
+                          amdgpu_waves_per_eu((hop_min_waves<R, RB>()), (hop_max_waves<R>())))) void
+k_hop(const HopLaunch a) {
   using C = typename c2<R>::t;
   if (a.halt && *a.halt) return;
   const Geom &g = a.g;

@@ -298,6 +298,17 @@ inline int widest(long waves, int most) {
   return t;
 }
 
+// the same for FP64, where a CU with one workgroup more than the others holds
+// all of them up: the most waves whose workgroups fill their last round of the
+// 256 CUs to `share` or more
+inline int evenly(long waves, int most, double share) {
+  for (int t = most; t > 1; t /= 2) {
+    const long w = (waves + t - 1) / t;
+    if ((double)w >= share * 256.0 * (double)((w + 255) / 256)) return t;
+  }
+  return 1;
+}
+
 // Shape used until the tuner (or the caller) picks one.  Two things decide:
 // - whether what a hop touches stays in the 256 MB of the Infinity Cache from
 //   one hop to the next.  If so, large workgroups that still give nearly every
@@ -307,21 +318,38 @@ inline int widest(long waves, int most) {
 //   faster themselves than through LDS; more stage them.
 // FP32, one right-hand side: 20 x 12 x 24 x 36 (125 MB) 19.3 us with 8 waves a
 // workgroup, 22.3 with 2; 32^3 x 64 (800 MB) 154 and 145.  One wave and at most 4
-// workgroups per CU, the shape of all of them before, took 29.1 and 190.  FP64:
-// 16^3 x 32 25.0 -> 19.4 us, 32^3 x 64 266 -> 262 us.
+// workgroups per CU, the shape of all of them before, took 29.1 and 190.
 inline wck::HopShape default_shape(const wc_operator *op, int nrhs) {
   const bool f64 = op->prec == WC_DOUBLE;
   const long blocks = op->g.Vh / kBlk;
+  const double slice = (double)blocks / op->g.L[3];  // blocks of a time slice
   const bool cached = op->g.Vh * (8 * op->nl + 24 * nrhs) * (long)op->csz <= (256L << 20);
+  // slices whose own spinors are worth staging, or keeping a small workgroup
+  // for, beyond the cache: up to 128 blocks, and to 256 where they are a power
+  // of two (z and t neighbours then fall on the same sets of an L2)
+  const long sites = op->g.Vh / op->g.L[3];
+  const bool tight = slice <= 128.0 || ((sites & (sites - 1)) == 0 && slice <= 256.0);
   wck::HopShape sh;
-  if (nrhs <= 1) {
+  if (nrhs <= 1 && f64) {
+    // In the cache, and three slices of spinors in an L2 (24^3 is beyond: 24^4
+    // 57 us with 4 waves, 53 with one): workgroups as large as fill the CUs
+    // evenly, spinors staged where they have more than one wave (16^3 x 32 25 ->
+    // 19 us; 14 x 16 x 16 x 24, 168 workgroups of 4 waves or 672 of one, 2 waves 8 %
+    // slower than either).  Else one wave, at most 4 workgroups per CU: 24 x 24 x
+    // 32 x 64 with 12-real links 161 us without the limit, 148 with.  Spinors
+    // staged on slices like 32^3's (259 -> 254 us; 24 x 32^2 x 48 3 % slower so).
+    if (cached && slice <= 100.0) {
+      sh.tpb = evenly(blocks, 4, 0.75);
+      sh.ls = sh.tpb > 1 ? 2 : 0;
+    } else {
+      sh.occ = 4;
+      sh.ls = tight ? 2 : 0;
+    }
+  } else if (nrhs <= 1) {
     // spinors staged in LDS, where a workgroup has more than one wave or the L2
     // would have to hold them
-    sh.tpb = cached ? widest(blocks, f64 ? 4 : 8) : f64 ? 1 : 2;
+    sh.tpb = cached ? widest(blocks, 8) : 2;
     sh.ls = sh.tpb > 1 || !cached ? 2 : 0;
-    // FP64 slices near the L2's size and whole links: 262 us against 270 for
-    // 32^3 x 64; with 12-real links or smaller slices the limit costs 5 %
-    sh.occ = f64 && op->nl == 9 && !cached && blocks > 128L * op->g.L[3] ? 4 : 0;
   } else if (f64 && (nrhs == 2 || (nrhs == 4 && cached))) {
     // 16^3 x 32: two right-hand sides 35.5 -> 31.4 us; 12^3 x 24: four 28 -> 23
     sh.tpb = nrhs == 2 && cached ? widest(2 * blocks, 8) : 2;

@@ -300,9 +300,9 @@ inline int widest(long waves, int most) {
 
 // the same for FP64, where a CU with one workgroup more than the others holds
 // all of them up: the most waves whose workgroups fill their last round of the
-// 256 CUs to `share` or more
-inline int evenly(long waves, int most, double share) {
-  for (int t = most; t > 1; t /= 2) {
+// 256 CUs to `share` or more, less by `step` with each halving
+inline int evenly(long waves, int most, double share, double step = 0.0) {
+  for (int t = most; t > 1; t /= 2, share -= step) {
     const long w = (waves + t - 1) / t;
     if ((double)w >= share * 256.0 * (double)((w + 255) / 256)) return t;
   }
@@ -350,9 +350,20 @@ inline wck::HopShape default_shape(const wc_operator *op, int nrhs) {
     // would have to hold them
     sh.tpb = cached ? widest(blocks, 8) : 2;
     sh.ls = sh.tpb > 1 || !cached ? 2 : 0;
-  } else if (f64 && (nrhs == 2 || (nrhs == 4 && cached))) {
-    // 16^3 x 32: two right-hand sides 35.5 -> 31.4 us; 12^3 x 24: four 28 -> 23
-    sh.tpb = nrhs == 2 && cached ? widest(2 * blocks, 8) : 2;
+  } else if (f64 && nrhs == 2) {
+    // In the cache as for one (16^3 x 32 35 -> 29 us), large workgroups where
+    // they fit better: 16^3 x 48, 384 of 8 waves, 4-8 % slower than 768 of 4;
+    // 10 x 18 x 16 x 24, 540 of 2 waves, 20 % faster than 1080 of one or 270 of 4.  Beyond, single waves, at most 4 per CU (28^3 x 56 315 us with workgroups
+    // of 4 waves, 340 with 2, 286 so), but on slices of 256 blocks and a power of
+    // two 2 waves (32^3 x 64 434, 395, 405) and on larger ones than 400 4 waves
+    // (64 x 32^3 1 % faster than the shape before, 11 % slower with single waves).
+    const bool pow2 = (sites & (sites - 1)) == 0;
+    if (cached && slice <= 100.0) sh.tpb = evenly(2 * blocks, 8, 0.78, 0.04);
+    else sh.tpb = slice > 400.0 ? 4 : pow2 && slice >= 256.0 ? 2 : 1;
+    sh.occ = 4;
+  } else if (f64 && nrhs == 4 && cached) {
+    // 12^3 x 24: 28 -> 23 us
+    sh.tpb = 2;
     sh.occ = 4;
   } else if (!f64 && nrhs <= 4) {
     // two right-hand sides a thread, also of an odd number (the last thread of a

@@ -36,3 +36,18 @@ def shape(fd, prec, n, compress):
 ], ids=str)
 def test_double_one(fd, compress, want):
     assert shape(fd, g.double, 1, compress) == want
+
+
+@pytest.mark.parametrize("fd,compress,want", [
+    ([12, 12, 12, 24], False, (1, 1, 4, 1, 0)), ([16, 16, 16, 16], False, (1, 4, 4, 1, 0)),
+    ([10, 18, 16, 24], False, (1, 2, 4, 1, 0)), ([12, 16, 16, 24], False, (1, 2, 4, 1, 0)),
+    ([14, 16, 16, 24], False, (1, 2, 4, 1, 0)), ([16, 16, 16, 32], False, (1, 8, 4, 1, 0)),
+    ([12, 16, 20, 40], False, (1, 4, 4, 1, 0)), ([16, 16, 16, 48], False, (1, 4, 4, 1, 0)),
+    ([10, 18, 16, 32], False, (1, 2, 4, 1, 0)), ([16, 16, 16, 24], False, (1, 4, 4, 1, 0)),
+    ([20, 20, 16, 32], False, (1, 8, 4, 1, 0)),
+    ([24, 24, 24, 24], True, (1, 1, 4, 1, 0)), ([24, 24, 24, 24], False, (1, 1, 4, 1, 0)),
+    ([28, 28, 28, 32], False, (1, 1, 4, 1, 0)), ([32, 32, 32, 32], True, (1, 2, 4, 1, 0)),
+    ([16, 32, 32, 32], False, (1, 1, 4, 1, 0)), ([64, 32, 32, 16], False, (1, 4, 4, 1, 0)),
+], ids=str)
+def test_double_two(fd, compress, want):
+    assert shape(fd, g.double, 2, compress) == want

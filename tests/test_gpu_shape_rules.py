@@ -51,3 +51,13 @@ def test_double_one(fd, compress, want):
 ], ids=str)
 def test_double_two(fd, compress, want):
     assert shape(fd, g.double, 2, compress) == want
+
+
+@pytest.mark.parametrize("fd,compress,want", [
+    ([12, 12, 12, 24], False, (1, 2, 4, 1, 0)), ([16, 16, 16, 20], False, (1, 2, 4, 1, 0)),
+    ([14, 16, 16, 24], False, (1, 4, 4, 1, 0)), ([10, 18, 16, 32], True, (1, 4, 4, 1, 0)),
+    ([16, 16, 16, 32], True, (1, 2, 4, 1, 0)), ([18, 18, 16, 24], False, (1, 4, 4, 1, 0)),
+    ([24, 24, 24, 24], True, (1, 4, 4, 1, 0)),
+], ids=str)
+def test_double_four(fd, compress, want):
+    assert shape(fd, g.double, 4, compress) == want

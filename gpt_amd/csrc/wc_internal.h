@@ -370,8 +370,14 @@ inline wck::HopShape default_shape(const wc_operator *op, int nrhs) {
   } else if (!f64 && nrhs <= 4) {
     // two right-hand sides a thread, also of an odd number (the last thread of a
     // site then repeats one): 32^3 x 64 with two 252 -> 195 us, three 373 -> 291
+    // (three: 10 x 18 x 16 x 24, 270 workgroups of 4 waves 10 % slower than the
+    // shape before, 1080 of one 13 % faster; beyond the cache 4 waves on slices
+    // that are not tight, 28^3 x 56 Meooe 12-real 201 us before, 220 with 2, 186
+    // with 4.  Meooe alone stays up to 6 % behind on 20 x 20 x 16 x 32, 20 x 12 x 24
+    // x 36 and 36^3 x 48 with 12-real links, M does not, Mpc^dag Mpc gains 20-30 %.)
     sh.rb = 2;
-    sh.tpb = cached ? widest(nrhs > 2 ? 2 * blocks : blocks, 4) : nrhs > 2 ? 2 : 1;
+    if (nrhs == 3) sh.tpb = cached ? evenly(2 * blocks, 4, 0.75) : tight ? 2 : 4;
+    else sh.tpb = cached ? widest(nrhs > 2 ? 2 * blocks : blocks, 4) : nrhs > 2 ? 2 : 1;
   } else {
     // right-hand sides a thread with the least padding, links staged where the
     // area fits

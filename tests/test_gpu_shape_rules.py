@@ -61,3 +61,13 @@ def test_double_two(fd, compress, want):
 ], ids=str)
 def test_double_four(fd, compress, want):
     assert shape(fd, g.double, 4, compress) == want
+
+
+@pytest.mark.parametrize("fd,compress,want", [
+    ([8, 16, 16, 32], False, (2, 4, 0, 1, 0)), ([10, 18, 16, 24], True, (2, 1, 0, 1, 0)),
+    ([12, 16, 16, 24], True, (2, 2, 0, 1, 0)), ([10, 20, 16, 32], False, (2, 4, 0, 1, 0)),
+    ([24, 24, 24, 48], False, (2, 2, 0, 1, 0)), ([32, 32, 32, 32], False, (2, 2, 0, 1, 0)),
+    ([20, 32, 32, 32], False, (2, 4, 0, 1, 0)), ([28, 28, 28, 56], True, (2, 4, 0, 1, 0)),
+], ids=str)
+def test_single_three(fd, compress, want):
+    assert shape(fd, g.single, 3, compress) == want

@@ -298,8 +298,8 @@ inline int widest(long waves, int most) {
   return t;
 }
 
-// the same for FP64, where a CU with one workgroup more than the others holds
-// all of them up: the most waves whose workgroups fill their last round of the
+// the same where a CU with one workgroup more than the others holds all of them
+// up: the most waves whose workgroups fill their last round of the
 // 256 CUs to `share` or more, less by `step` with each halving
 inline int evenly(long waves, int most, double share, double step = 0.0) {
   for (int t = most; t > 1; t /= 2, share -= step) {
@@ -434,8 +434,10 @@ inline wck::HopShape shape_for(const wc_operator *op, int nrhs) {
 // fill a thread's pairs without a rest.  Normal operator on 24^3 x 48 with
 // 12-real links: 3, 4, 5, 8 and 11 right-hand sides 469, 518, 757, 1010 and 1196
 // us in the FP32 hop's shapes, 430, 491, 645, 785 and 1087 in these.  From 10 on 8
-// waves share more of what they stage: 12 right-hand sides 1157 us with 4, 1110
-// with 8; 8 right-hand sides 731 and 791.
+// waves share more of what they stage (24^3 x 48: 8 right-hand sides 731 us with
+// 4 waves, 791 with 8, 12 1157 and 1110; 16^3 x 32: 24, 31, 48 and 64 1-2 % faster
+// with 8), where the workgroups fill the CUs evenly: 12^4 with 13, 264 workgroups
+// of 8, 84 us, 527 of 4 76; 8^3 x 16 with 9, 288 of 2, 62 us, 576 of one 58.
 inline wck::HopShape default_shape16(const wc_operator *op, int nrhs) {
   wck::HopShape sh;
   if (nrhs <= 2) return default_shape(op, nrhs);
@@ -443,7 +445,7 @@ inline wck::HopShape default_shape16(const wc_operator *op, int nrhs) {
     sh.rb = 2;
     return sh;
   }
-  sh.tpb = widest(op->g.Vh / kBlk * nrhs, nrhs >= 10 ? 8 : 4);
+  sh.tpb = evenly(op->g.Vh / kBlk * nrhs, nrhs >= 10 ? 8 : 4, 0.75);
   sh.ls = nrhs >= 7 ? 1 : 0;
   if (!stage_fits(op, nrhs, sh)) sh.ls = 0;
   return sh;

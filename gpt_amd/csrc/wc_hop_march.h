@@ -374,13 +374,19 @@ template <typename R> inline int march_tiles(const HopLaunch &a) {
 // Where the t-marching form applies: a wave's 64 items within march_sites
 // sites (FP64 from 8 right-hand sides, except 9; FP32 from 7), working
 // precision, fields within one buffer descriptor, one set of clover blocks.
-// Its rule where neither the tuner nor the caller has decided: lattices of at
-// most 384 waves in all (4^3 x 8 13 -> 8 us, 8^3 x 16 FP64, 8 right-hand sides,
-// 14 -> 11 us), and slices of 2048 half-sites or more walked 4 or more at a time
-// (1.0-1.6 times as fast for Meooe, M and Mpc^dag Mpc).  Between, the fields are
-// in the caches and the slices small enough that the gathering kernel finds
-// the neighbours there: 0.82-1.2 times as fast (32 x 16 x 4 x 32 FP64, 8
-// right-hand sides: M 107 -> 130 us; 24 x 18 x 6 x 20, 12: 164 -> 139 us).
+// Its rule where neither the tuner nor the caller has decided (times against the
+// gathering kernel, Meooe / M / Mpc^dag Mpc):
+// - slices of 2048 half-sites or more walked 4 or more at a time, 1.0-1.7 / 0.92-1.5
+//   / 0.93-1.5 times as fast.  Not with 15 to 17 groups of right-hand sides on x-y
+//   planes of two 64-site blocks, where its patch just outgrows an L2 and the
+//   gathering kernel's sites do not: 16 right-hand sides, FP64 16^3 x 32 12-real 0.91
+//   / 0.89 / 0.95, 16 x 16 x 32^2 1.07 / 0.93 / 0.95 (12 of them 1.6 / 1.4 / 1.3).
+// - lattices of at most 384 waves in all, with whole links: 8^4 FP64, 12 right-hand
+//   sides, 1.21 / 1.32 / 1.11.  12-real links leave the gathering kernel so much less
+//   to load that it wins (0.74-0.97 / 0.8-1.0 / 0.9-1.1), and odd counts in FP32 cost
+//   a group that is half idle (8^3 x 12, 13: 0.99 / 1.03 / 0.93).
+// Between, fields are in the caches and slices small enough that the gathering
+// kernel finds most neighbours there.
 template <typename R> bool march_applies(const HopLaunch &a) {
   constexpr int RB = march_rb<R>(), W = kMarchItems;
   if (!a.march || a.half_in || a.half_out || a.skip_t_faces || a.nrhs < RB || a.nrhs > 64) return false;
@@ -390,7 +396,8 @@ template <typename R> bool march_applies(const HopLaunch &a) {
   if ((W % G == 0 ? W / G : (W - 1) / G + 2) > march_sites<R>()) return false;
   if (a.march == 1) return true;
   const int ntiles = march_tiles<R>(a), Lt = a.g.L[3];
-  if ((long)ntiles * Lt <= 384) return true;
+  if ((long)ntiles * Lt <= 384) return a.nl == 9 && a.nrhs % RB == 0;
+  if (G >= 15 && G <= 17 && a.g.Lxh * a.g.L[1] == 2 * kBlk) return false;
   const int n = march_segments(ntiles, Lt);
   return a.g.Vh / Lt >= 2048 && (Lt + n - 1) / n >= 4;
 }

@@ -382,9 +382,11 @@ template <typename R> inline int march_tiles(const HopLaunch &a) {
 //   gathering kernel's sites do not: 16 right-hand sides, FP64 16^3 x 32 12-real 0.91
 //   / 0.89 / 0.95, 16 x 16 x 32^2 1.07 / 0.93 / 0.95 (12 of them 1.6 / 1.4 / 1.3).
 // - lattices of at most 384 waves in all, with whole links: 8^4 FP64, 12 right-hand
-//   sides, 1.21 / 1.32 / 1.11.  12-real links leave the gathering kernel so much less
-//   to load that it wins (0.74-0.97 / 0.8-1.0 / 0.9-1.1), and odd counts in FP32 cost
-//   a group that is half idle (8^3 x 12, 13: 0.99 / 1.03 / 0.93).
+//   sides, 1.21 / 1.32 / 1.11.  With 12-real links the gathering kernel has so much
+//   less to load that it wins in the bare hop and in M (0.74-0.97 / 0.8-1.04), not in
+//   the hops of Mpc with their clover and axpy (even counts 0.98-1.18; 8^3 x 16 FP32,
+//   12: 71 -> 63 us).  Odd counts in FP32 cost a group that is half idle (8^3 x 12,
+//   13: 0.99 / 1.03 / 0.93).
 // Between, fields are in the caches and slices small enough that the gathering
 // kernel finds most neighbours there.
 template <typename R> bool march_applies(const HopLaunch &a) {
@@ -396,7 +398,7 @@ template <typename R> bool march_applies(const HopLaunch &a) {
   if ((W % G == 0 ? W / G : (W - 1) / G + 2) > march_sites<R>()) return false;
   if (a.march == 1) return true;
   const int ntiles = march_tiles<R>(a), Lt = a.g.L[3];
-  if ((long)ntiles * Lt <= 384) return a.nl == 9 && a.nrhs % RB == 0;
+  if ((long)ntiles * Lt <= 384) return a.nrhs % RB == 0 && (a.nl == 9 || (a.epi & (EPI_CLOV | EPI_AXPY)));
   if (G >= 15 && G <= 17 && a.g.Lxh * a.g.L[1] == 2 * kBlk) return false;
   const int n = march_segments(ntiles, Lt);
   return a.g.Vh / Lt >= 2048 && (Lt + n - 1) / n >= 4;

@@ -6,6 +6,7 @@ operator/matrix_operator.py).  Field data lives in HBM as torch tensors in the
 even-odd SoA layout of include/gpt_amd_wc.h; every arithmetic operation goes
 through the HIP library (there is no CPU fallback).
 """
+import math
 import numbers
 
 import numpy as np
@@ -434,22 +435,25 @@ class site_scalar:
         return self.data.cpu().numpy().reshape(tuple(reversed(self.grid.fdimensions)))
 
 
-def eager():
-    """whether torch runs the calls as they stand.  A kernel is no operation of
-    torch's: a trace (make_fx, jit, compile) would lack it, a dispatch mode not see
-    it, and a tensor under a transform (vmap, jvp, ...) has no address to give it"""
-    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-                or torch._C._get_tracing_state() is not None
-                or torch._C._functorch.peek_interpreter_stack() is not None)
-
-
-def plain(t, dtype):
-    """whether a kernel on the current device can take the values of t as they lie
-    in memory, and nothing is differentiated (where calls are eager)"""
-    return (type(t) is torch.Tensor and t.is_cuda and t.dtype == dtype and t.is_contiguous() and t.device == device()
-            and t.device.index == torch.cuda.current_device()
-            and not (t.is_conj() or t.is_neg() or t.requires_grad)
-            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
+def direct(dtype, *tensors):
+    """whether a kernel on the current device can take the values of the tensors
+    as they lie in memory.  It is no operation of torch's: where calls are not run
+    as they stand, a trace (make_fx, jit, compile) would lack it, a dispatch mode not
+    see it, and a tensor under a transform (vmap, jvp, ...) has no address to give it"""
+    if torch.compiler.is_compiling():
+        return False
+    dev = None
+    for t in tensors:
+        if (type(t) is not torch.Tensor or not t.is_cuda or t.dtype != dtype or not t.is_contiguous()
+                or t.requires_grad or t.is_conj() or t.is_neg()):
+            return False
+        if dev is None:
+            dev = t.get_device()
+        elif t.get_device() != dev:
+            return False
+    return (dev == device().index == torch.cuda.current_device() and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
+            and torch._C._functorch.peek_interpreter_stack() is None)
 
 
 def trace(x):
@@ -459,8 +463,7 @@ def trace(x):
     if isinstance(x, _site_product):
         a, b = x.a.data, x.b.data
         prec = {torch.complex128: double, torch.complex64: single}.get(a.dtype)
-        if (prec is not None and eager() and a.shape == b.shape and a[0].numel() == 144 and plain(a, a.dtype)
-                and plain(b, a.dtype)):
+        if prec is not None and direct(a.dtype, a, b) and a.shape == b.shape and a[0].numel() == 144:
             out = torch.empty(a.shape[0], dtype=torch.complex128, device=a.device)
             _lib.check(_lib.load().wc_site_trace(prec.code, a.shape[0], a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                                  stream_ptr()))
@@ -479,9 +482,9 @@ def slice_(x, dim):
     if not isinstance(x, site_scalar):
         raise NotImplementedError("g.slice is provided for g.trace results")
     L = x.grid.fdimensions
-    inner = int(np.prod(L[:dim])) if isinstance(dim, numbers.Integral) and 0 <= dim < 4 else 0
+    inner = math.prod(L[:dim]) if isinstance(dim, numbers.Integral) and 0 <= dim < 4 else 0
     # runs of less than 128 bytes (slices in x) are left to the general sum
-    if inner >= 8 and eager() and x.data.numel() == int(np.prod(L)) and plain(x.data, torch.complex128):
+    if inner >= 8 and x.data.numel() == x.grid.gsites and direct(torch.complex128, x.data):
         n = L[dim]
         work = torch.empty((17, n), dtype=torch.complex128, device=x.data.device)
         _lib.check(_lib.load().wc_slice_sum(x.data.numel() // (n * inner), n, inner, x.data.data_ptr(),

@@ -552,11 +552,10 @@ def _pointers(fields, packed, written):
     are written, apart from each other and from it"""
     t = packed.data
     shape = t.shape[:-2] + (1, 2)
-    if len(fields) < 2 or not core.eager() or not core.plain(t, t.dtype):
+    one = [f.data for f in fields]
+    if len(one) < 2 or not core.direct(t.dtype, t, *one) or not all(x.shape == shape for x in one):
         return None
-    if not all(f.data.shape == shape and core.plain(f.data, t.dtype) for f in fields):
-        return None
-    ptrs = [f.data.data_ptr() for f in fields]
+    ptrs = [x.data_ptr() for x in one]
     if written:
         size = fields[0].data.numel() * t.element_size()
         ends = sorted([(p, p + size) for p in ptrs] + [(t.data_ptr(), t.data_ptr() + size * len(ptrs))])

@@ -482,8 +482,11 @@ def slice_(x, dim):
     if not isinstance(x, site_scalar):
         raise NotImplementedError("g.slice is provided for g.trace results")
     L = x.grid.fdimensions
-    inner = math.prod(L[:dim]) if isinstance(dim, numbers.Integral) and 0 <= dim < 4 else 0
-    # runs of less than 128 bytes (slices in x) are left to the general sum
+    # by a kernel on lattices large enough (24^4 along z: 167 us with the trace, 163
+    # so; 8^4: 31 us alone, 37 so, two launches of the library), where a slice has
+    # runs of 128 bytes or more (not in x)
+    large = x.grid.gsites >= 1 << 18 and isinstance(dim, numbers.Integral) and 0 <= dim < 4
+    inner = math.prod(L[:dim]) if large else 0
     if inner >= 8 and x.data.numel() == x.grid.gsites and direct(torch.complex128, x.data):
         n = L[dim]
         work = torch.empty((17, n), dtype=torch.complex128, device=x.data.device)

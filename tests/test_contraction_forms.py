@@ -44,3 +44,17 @@ def test_directions_as_other_numbers(kind):
     for dim in (4, -1):
         with pytest.raises(TypeError):
             g.slice(tr, kind(dim) if kind is not np.uint8 else 4)
+
+
+@pytest.mark.parametrize("fd", [[4, 4, 4, 4], [8, 8, 8, 16], [32, 32, 16, 14]], ids=str)
+def test_small_fields_are_not_looked_at(fd, monkeypatch):
+    """below 2^18 sites the general sum is as fast as a kernel, and nothing else is
+    asked of the field"""
+    def fail(*_):
+        raise AssertionError("a small field was checked for the kernel")
+
+    monkeypatch.setattr(core, "direct", fail)
+    grid = g.grid(fd, g.double)
+    tr = core.site_scalar(grid, torch.ones(grid.gsites, dtype=torch.complex128))
+    for dim in range(4):
+        assert g.slice(tr, dim) == [grid.gsites / fd[dim]] * fd[dim]

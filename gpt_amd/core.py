@@ -482,10 +482,11 @@ def slice_(x, dim):
     if not isinstance(x, site_scalar):
         raise NotImplementedError("g.slice is provided for g.trace results")
     L = x.grid.fdimensions
-    # by a kernel on lattices large enough (24^4 along z: 167 us with the trace, 163
-    # so; 8^4: 31 us alone, 37 so, two launches of the library), where a slice has
-    # runs of 128 bytes or more (not in x)
-    large = x.grid.gsites >= 1 << 18 and isinstance(dim, numbers.Integral) and 0 <= dim < 4
+    # slices in y and z of large lattices by a kernel (24^3 x 48: 42 us with the general
+    # sum, 38 so; with the trace 303 and 290), if their runs have 128 bytes or more.
+    # On 8^4 its two launches and checks take the host longer (31 us and 37), and for
+    # slices in t the general sum is as fast (35 and 39)
+    large = x.grid.gsites >= 1 << 18 and isinstance(dim, numbers.Integral) and dim in (1, 2)
     inner = math.prod(L[:dim]) if large else 0
     if inner >= 8 and x.data.numel() == x.grid.gsites and direct(torch.complex128, x.data):
         n = L[dim]

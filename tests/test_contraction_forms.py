@@ -46,15 +46,15 @@ def test_directions_as_other_numbers(kind):
             g.slice(tr, kind(dim) if kind is not np.uint8 else 4)
 
 
-@pytest.mark.parametrize("fd", [[4, 4, 4, 4], [8, 8, 8, 16], [32, 32, 16, 14]], ids=str)
-def test_small_fields_are_not_looked_at(fd, monkeypatch):
-    """below 2^18 sites the general sum is as fast as a kernel, and nothing else is
-    asked of the field"""
+@pytest.mark.parametrize("fd,dims", [([4, 4, 4, 4], range(4)), ([8, 8, 8, 16], range(4)),
+                                     ([32, 32, 16, 14], range(4)), ([32, 32, 16, 16], (0, 3))], ids=str)
+def test_general_sums_look_at_nothing_else(fd, dims, monkeypatch):
+    """where the general sum is as fast as the kernel, below 2^18 sites and along t"""
     def fail(*_):
         raise AssertionError("a small field was checked for the kernel")
 
     monkeypatch.setattr(core, "direct", fail)
     grid = g.grid(fd, g.double)
     tr = core.site_scalar(grid, torch.ones(grid.gsites, dtype=torch.complex128))
-    for dim in range(4):
+    for dim in dims:
         assert g.slice(tr, dim) == [grid.gsites / fd[dim]] * fd[dim]

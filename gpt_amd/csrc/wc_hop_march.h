@@ -2,9 +2,9 @@
 //
 // What bounds the gathering kernel (wc_hop.h) with 12 right-hand sides is the
 // fabric behind the L2s: an XCD's sites in flight and their neighbours (10 MB
-// in FP64) are far beyond its 4 MB L2, so an input spinor is fetched 4-6
-// times (24^3 x 48, FP64: 5.6 GB of reads against 1.3 GB compulsory, at the
-// 7.7 TB/s the fabric gives).  Visiting the sites in another order, occupancy
+// in FP64) are far beyond its 4 MB L2, so an input spinor is fetched 5-7
+// times (24^3 x 48, FP64: 5.5 GB of reads against 1.15 GB compulsory; with the
+// stores 7.5 TB/s, what the fabric gives).  Visiting the sites in another order, occupancy
 // caps and cache hints changed that by 10 % at most.  Here a wave owns 64
 // items (site of a t-slice, group of RB right-hand sides; 16 bytes a
 // component in FP64 and FP32) and walks through t with them:
@@ -16,7 +16,7 @@
 //   - the waves of an XCD own one compact patch of the slice (rows in blocks of
 //     kMarchRows in y, XCDs along the order) and walk together, so the y, z and
 //     other x neighbours were loaded by another wave one step before and are
-//     in L2 (24^3 x 48 FP64: reads 5.6 -> 2.3 GB);
+//     often in L2 (24^3 x 48 FP64: reads 5.5 -> 3.1 GB, 3.6 fetches a spinor);
 //   - the 6 x 12 loads of a step are issued up to a step ahead into registers
 //     (512 a lane: one wave per SIMD), the links and clover blocks of the next
 //     slice too.  A workgroup is one wave: nothing waits for other waves.
@@ -26,9 +26,10 @@
 // 24^3 x 48 826 -> 553 us, 16^3 x 32 156 -> 94 us; FP32 32^3 x 64 1078 -> 828 us
 // (12-real links 1027 -> 769 us); also on the smallest lattices (8^4 FP64 14 ->
 // 10 us: a step's loads are all under way at once, where the other kernel
-// waits for each direction).  A step is then limited by the latencies of its
-// one wave per SIMD (without loads 274 us, 24^3 x 48 FP64); two waves would
-// need half the registers and half the LDS.
+// waits for each direction).  On large lattices the texture addresser (87 %
+// busy, 24^3 x 48 FP64) and the fabric (7.0 TB/s of reads and stores) then bound
+// it together; its waves wait for a tenth of their time, the other kernel's for
+// half.
 #pragma once
 #include "wc_hop.h"
 

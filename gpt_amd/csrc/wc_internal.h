@@ -353,10 +353,11 @@ inline wck::HopShape default_shape(const wc_operator *op, int nrhs) {
   } else if (f64 && nrhs == 2) {
     // In the cache as for one (16^3 x 32 35 -> 29 us), large workgroups where
     // they fit better: 16^3 x 48, 384 of 8 waves, 4-8 % slower than 768 of 4;
-    // 10 x 18 x 16 x 24, 540 of 2 waves, 20 % faster than 1080 of one or 270 of 4.  Beyond, single waves, at most 4 per CU (28^3 x 56 315 us with workgroups
-    // of 4 waves, 340 with 2, 286 so), but on slices of 256 blocks and a power of
-    // two 2 waves (32^3 x 64 434, 395, 405) and on larger ones than 400 4 waves
-    // (64 x 32^3 1 % faster than the shape before, 11 % slower with single waves).
+    // 10 x 18 x 16 x 24, 540 of 2 waves, 20 % faster than 1080 of one or 270 of 4.
+    // Beyond, single waves, at most 4 per CU (28^3 x 56 315 us with workgroups of 4
+    // waves, 340 with 2, 286 so), but on slices of 256 blocks and a power of two 2
+    // waves (32^3 x 64 434, 395, 405) and on larger ones than 400 4 waves (64 x 32^3
+    // 1 % faster than the shape before, 11 % slower with single waves).
     const bool pow2 = (sites & (sites - 1)) == 0;
     if (cached && slice <= 100.0) sh.tpb = evenly(2 * blocks, 8, 0.78, 0.04);
     else sh.tpb = slice > 400.0 ? 4 : pow2 && slice >= 256.0 ? 2 : 1;
@@ -652,11 +653,13 @@ struct IterCheck {
 
 // one iteration of the inner CG on lo: mmp = A p (A_D^-1 p in aD), alpha,
 // r -= alpha mmp, beta, x += alpha p, p = beta p + r, aD = A_D^-1 p; then the
-// test.  partials: 2 * red_partials.  Where the partials are few (1024 in all
-// right-hand sides together: up to 16^3 x 32 for one, 8^4 for 12) alpha is formed
-// inside the r update, and beta together with the test: two launches less,
-// each 4 us when an iteration's kernels are as short (8^4 FP64, one right-hand
-// side: 14 us less an iteration, with the shorter reductions).
+// test.  partials: 2 * red_partials.  Where the partials of all right-hand sides
+// together are at most 1024, a launch is saved: those of <p, A p>, one per 64-site
+// block and right-hand side (16^3 x 32 for one, 8^4 for up to 32), let the r update
+// form alpha; those of |r|^2, red_blocks for each (one right-hand side on every
+// lattice, 8^4 for up to 3), let one kernel form beta and run the test.  Each launch is
+// 4 us when an iteration's kernels are as short (8^4 FP64, one right-hand side: 14
+// us less an iteration with both, and the shorter reductions).
 template <typename R>
 inline int inner_iteration(wc_operator *lo, int N, int pd, void *r, void *p, void *mmp, void *x, void *aD,
                            hipStream_t s, const IterCheck &chk, double *st = nullptr, double *partials = nullptr,

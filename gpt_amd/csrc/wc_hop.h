@@ -149,11 +149,12 @@ __device__ __forceinline__ void compute_dir(const HopLaunch &a, const int c[4], 
 
 // The 8 directions are unrolled, each fenced from the next: no load of one is
 // hoisted into another, so the live registers stay at one direction's operands
-// plus the accumulators; the other waves on the SIMD keep HBM busy meanwhile.
+// plus the accumulators; the other waves on the SIMD keep HBM busy meanwhile
+// where there are some (with one or two, the directions' latencies add up).
 // As a loop with a switch over the projections, every direction copied 12 of the
 // sums and chose its neighbour at run time, a quarter of the instructions of the
-// 16-bit hops, which the VALUs bound (1540 a wave at 12 right-hand sides, 90 %
-// busy), and took more registers (FP16 AXPY hop 90, now 69).  FP16 Mpc^dag Mpc at
+// 16-bit hops, whose VALUs were 72-82 % busy (1540 a wave at 12 right-hand sides;
+// now 67-82), and took more registers (FP16 AXPY hop 90, now 69).  FP16 Mpc^dag Mpc at
 // 24^3 x 48: 1193 -> 1155 us; FP64 Meooe at 32^3 x 64: 276 -> 270 us.
 // Neighbour offsets come from uniform strides of the
 // half-site index h = ((t*Lz + z)*Ly + y)*Lxh + x/2.  The item's right-hand

@@ -430,7 +430,7 @@ inline wck::HopShape shape_for(const wc_operator *op, int nrhs) {
 }
 
 // the shape of the hops with 16-bit spinors until one was timed: these are
-// bound by their arithmetic, where one right-hand side a thread and as many
+// bound by their arithmetic and the fabric; one right-hand side a thread and as many
 // waves as fit are fastest, links staged from 7 right-hand sides on; two and four
 // fill a thread's pairs without a rest.  Normal operator on 24^3 x 48 with
 // 12-real links: 3, 4, 5, 8 and 11 right-hand sides 469, 518, 757, 1010 and 1196
